@@ -117,6 +117,11 @@ size_t skinny_m_workspace(const GemmArgs& g);
 // of 64, enough rows): faster than the split-precision kernels there.
 bool f32_takes_w112(const GemmArgs& g);
 int launch_gemm_narrow(const GemmArgs& g, hipStream_t stream);
+// FP32 products from three exact bf16 parts per operand (gemm_parts.hip):
+// the plain output map, enough rows and columns for its tiles, K up to 2^16.
+bool gemm_parts_ok(const GemmArgs& g);
+size_t gemm_parts_workspace(const GemmArgs& g);
+int launch_gemm_parts(const GemmArgs& g, hipStream_t stream);
 int launch_dgemm(int opA, int opB, int64_t M, int64_t N, int64_t K,
                  const double* A, int64_t lda, const double* B, int64_t ldb,
                  double* C, int64_t ldc, hipStream_t stream);
