@@ -102,6 +102,9 @@ inline GemmArgs with_ones_column(GemmArgs g) {
 // configuration choice.
 int launch_gemm_f32(const GemmArgs& g, hipStream_t stream);
 size_t gemm_f32_workspace(const GemmArgs& g);
+// (its tiled kernels alone, gemm_f32.hip)
+int launch_gemm_f32_tiled(const GemmArgs& g, hipStream_t stream);
+size_t gemm_f32_tiled_workspace(const GemmArgs& g);
 size_t gemm_bf16x3_workspace(const GemmArgs& g, int terms);
 // terms = 3 (bf16x3: hi*hi + hi*lo + lo*hi) or 4 (adds lo*lo).
 int launch_gemm_bf16x3(const GemmArgs& g, int terms, hipStream_t stream);
@@ -122,6 +125,12 @@ int launch_gemm_narrow(const GemmArgs& g, hipStream_t stream);
 bool gemm_parts_ok(const GemmArgs& g);
 size_t gemm_parts_workspace(const GemmArgs& g);
 int launch_gemm_parts(const GemmArgs& g, hipStream_t stream);
+// FP32 products too small for the tiled kernels' workgroups, operands read
+// straight from global memory (gemm_direct.hip; either output map, batches,
+// ones column, no workspace).
+bool gemm_direct_ok(const GemmArgs& g);
+bool gemm_direct_for_tf32(const GemmArgs& g);
+int launch_gemm_direct(const GemmArgs& g, hipStream_t stream);
 int launch_dgemm(int opA, int opB, int64_t M, int64_t N, int64_t K,
                  const double* A, int64_t lda, const double* B, int64_t ldb,
                  double* C, int64_t ldc, hipStream_t stream);

@@ -83,11 +83,11 @@ int dispatch16(const GemmArgs& g, hipStream_t stream) {
 // dX) take it in the TF32 modes too: 35.5 against 40.2 us there, with exact
 // products (inside the TF32-mode error bar).
 static bool to_f32(const GemmArgs& g, int terms) {
-    return narrow_kind(g) || tn_split_to_f32(g, terms) || f32_takes_w112(g);
+    return narrow_kind(g) || tn_split_to_f32(g, terms) || f32_takes_w112(g) ||
+           gemm_direct_for_tf32(g);
 }
 
-size_t gemm_bf16x3_workspace(const GemmArgs& g, int terms) {
-    if (to_f32(g, terms)) return gemm_f32_workspace(g);
+static size_t bf_workspace(const GemmArgs& g, int terms) {
     switch (choose_bf(g, terms)) {
         case BfCfg::SkinnyM: return ws_of<CfgSkinnyM>(g);
         case BfCfg::Huge: return ws_of<CfgHuge>(g);
@@ -96,6 +96,13 @@ size_t gemm_bf16x3_workspace(const GemmArgs& g, int terms) {
         case BfCfg::Large: return ws_of<CfgLarge>(g);
         default: return ws_of<CfgSmall>(g);
     }
+}
+
+size_t gemm_bf16x3_workspace(const GemmArgs& g, int terms) {
+    // a query knows neither alignment nor leading dimensions, on which the
+    // route depends: enough for either
+    const size_t f32 = to_f32(g, terms) ? gemm_f32_workspace(g) : 0, bf = bf_workspace(g, terms);
+    return f32 > bf ? f32 : bf;
 }
 
 // Products with K <= 16 or N <= 16 (narrow_kind) take the FP32 narrow

@@ -288,19 +288,13 @@ static size_t cfg_workspace(const GemmArgs& g, F32Cfg c) {
     }
 }
 
-size_t gemm_f32_workspace(const GemmArgs& g) {
-    if (const int nk = narrow_kind(g)) return nk == 3 ? skinny_m_workspace(g) : 0;
+size_t gemm_f32_tiled_workspace(const GemmArgs& g) {
     bool blocked;
     const F32Cfg c = choose_f32(g, blocked);
-    if (blocked) return 0;
-    // a query knows no leading dimensions: enough for either route
-    const size_t parts = gemm_parts_ok(g) ? gemm_parts_workspace(g) : 0, own = cfg_workspace(g, c);
-    return parts > own ? parts : own;
+    return blocked ? 0 : cfg_workspace(g, c);
 }
 
-int launch_gemm_f32(const GemmArgs& g, hipStream_t stream) {
-    if (narrow_kind(g)) return launch_gemm_narrow(g, stream);
-    if (gemm_parts_ok(g)) return launch_gemm_parts(g, stream);
+int launch_gemm_f32_tiled(const GemmArgs& g, hipStream_t stream) {
     bool blocked;
     const F32Cfg c = choose_f32(g, blocked);
     int64_t full = 0;
