@@ -424,6 +424,15 @@ int64_t own_tiles(const GemmArgs& g) {
     return ceil_div(g.M, PTile::BM) * ceil_div(nb, PTile::BN);
 }
 
+// The tile count that the k-slices are chosen for: that of the tiled kernel's
+// 128 x 64 slice tiles where it would split too, so that both routes take the
+// same slices (and ask for the same workspace).
+int64_t slice_tiles(const GemmArgs& g) {
+    const int64_t nb = g.ones_col >= 0 ? g.ones_col : g.N;
+    const int64_t t = ceil_div(g.M, 128) * ceil_div(nb, 64);
+    return splitk_applies(t, g.K) ? t : own_tiles(g);
+}
+
 }  // namespace
 
 // Which products: those with a 128 x 128 tile for nearly every CU (2048^3 92
@@ -444,13 +453,13 @@ bool gemm_parts_ok(const GemmArgs& g) {
     return tiles >= 240 || (g.batch == 1 && splitk_applies(tiles, g.K));
 }
 
-size_t gemm_parts_workspace(const GemmArgs& g) { return splitk_bytes(g, own_tiles(g), PBK); }
+size_t gemm_parts_workspace(const GemmArgs& g) { return splitk_bytes(g, slice_tiles(g), PBK); }
 
 int launch_gemm_parts(const GemmArgs& g0, hipStream_t stream) {
     const int64_t tiles = ceil_div(g0.M, PTile::BM) * ceil_div(g0.N, PTile::BN);
     if (tiles > INT32_MAX) return set_error(CDX_ERR_UNSUPPORTED, "gemm: too many tiles");
     if (g0.batch < 1 || g0.batch > 65535) return set_error(CDX_ERR_UNSUPPORTED, "gemm: batch out of range");
-    return with_splitk(g0, own_tiles(g0), PBK, stream,
+    return with_splitk(g0, slice_tiles(g0), PBK, stream,
                        [&](const GemmArgs& g, int splits, int64_t k_chunk) {
         const KParams kp = f32::kparams_of(g, k_chunk);
         const dim3 grid((unsigned)tiles, (unsigned)splits, (unsigned)g.batch), block(PTile::NT);
