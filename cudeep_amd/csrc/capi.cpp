@@ -178,21 +178,66 @@ size_t col_round_bytes(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int64_
     return per * (size_t)col_round_images(batch, per, S);
 }
 
-// The reference's forward dispatch (conv_kernel.cu:242-275) below its
-// Winograd route: a layer whose column buffer would exceed 4 MiB runs the
-// implicit GEMM (no buffer) unless it is a 3x3 stride-1 layer with >= 16
-// output pixels per image (the Winograd shape, which keeps the im2col route
-// here when it is not sent to Winograd).  The reference's naive-kernel
-// shapes (K_col < 9 or fewer than 4 output pixels per image, checked before
-// the implicit route at conv_kernel.cu:250) take the im2col route, which
-// computes the same sums.
+bool forward_few_columns(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int64_t KH, int64_t KW,
+                         int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
+    return col_bytes(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW) <= ((size_t)4 << 20);
+}
+
+// The forward dispatch below the Winograd route.  The reference sends a layer
+// whose column buffer would exceed 4 MiB to its implicit kernel (no buffer;
+// conv_kernel.cu:242-275); here every layer takes the implicit GEMM unless it
+// is a 3x3 stride-1 layer with >= 16 output pixels per image (the Winograd
+// shape, which keeps the im2col route here when it is not sent to Winograd):
+// below 4 MiB of columns one launch beats im2col + GEMM as well (6 x 56 -> 46,
+// 31^2, 3x3 stride 2: 16 -> 11 us; 3 x 168 -> 99, 56^2, 1x1 stride 2: 13 ->
+// 9), and its products are fp32 in every precision mode.  The reference's
+// naive-kernel shapes (K_col < 9 or fewer than 4 output pixels per image,
+// checked before the implicit route at conv_kernel.cu:250) take the im2col
+// route, which computes the same sums.
 bool forward_takes_implicit(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int64_t KH,
                             int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
     const int64_t OH = conv_out(IH, KH, SH, PH), OW = conv_out(IW, KW, SW, PW);
-    if (KH == 3 && KW == 3 && SH == 1 && SW == 1 && OH * OW >= 16) return false;
+    const bool s3 = KH == 3 && KW == 3 && SH == 1 && SW == 1;
+    if (s3 && (OH * OW >= 16 || forward_few_columns(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW)))
+        return false;
     if (IC * KH * KW < 9 || OH * OW < 4) return false;
-    return col_bytes(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW) > ((size_t)4 << 20) &&
-           cdx::conv_fwd_implicit_ok(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW);
+    return cdx::conv_fwd_implicit_ok(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW);
+}
+
+// The workspace a forward call asks for: one round of columns, except that of
+// layers whose whole column buffer would exceed 4 MiB and that never form it.
+// (Layers of fewer columns that no longer form them keep asking for it, so
+// that a caller's check of the size stays what it was.)
+size_t forward_workspace(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int64_t KH, int64_t KW,
+                         int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
+    if (!forward_few_columns(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW) &&
+        forward_takes_implicit(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW))
+        return 0;
+    return col_round_bytes(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW);
+}
+
+// A 1x1 convolution with stride 1 and no padding is a product per image of the
+// tensors as they lie, with no columns to form: y_b [OC, S] = w [OC, IC] x_b
+// [IC, S], dx_b = w^T dy_b (the filter transposed first, and the sum over
+// output channels in two levels, as the row-window kernel does).  FP32
+// products in every precision mode, as on the implicit route these layers took
+// beyond 4 MiB of columns (16 x 256 -> 64 channels at 56^2: forward 63 -> 24
+// us, backward data 51 -> 28; 14 x 53 -> 64 at 60^2: 22 -> 14, 24 -> 16).
+bool conv_is_product(int64_t batch, int64_t IC, int64_t OC, int64_t KH, int64_t KW, int64_t SH,
+                     int64_t SW, int64_t PH, int64_t PW) {
+    return KH == 1 && KW == 1 && SH == 1 && SW == 1 && PH == 0 && PW == 0 && IC > 0 && OC > 0 &&
+           batch <= 65535;
+}
+
+int conv_product(const float* w, int64_t rows, int64_t depth, const float* in, const float* bias,
+                 float* out, int64_t batch, int64_t S, bool two_level, hipStream_t stream) {
+    cdx::GemmArgs g{CDX_OP_N, CDX_OP_N, rows, S, depth, w, depth, in, S, out, S, 0, 0, bias,
+                    bias ? CDX_BIAS_ROW : CDX_BIAS_NONE, CDX_EPI_NONE};
+    g.batch = batch;
+    g.stride_b = depth * S;
+    g.stride_c = rows * S;
+    g.blocked_sum = two_level;
+    return cdx::launch_gemm_f32(g, stream);
 }
 
 }  // namespace
@@ -380,11 +425,8 @@ size_t cdx_conv2d_forward_workspace_size(int64_t batch, int64_t in_channels, int
     if (check_conv("cdx_conv2d_forward_workspace_size", batch, in_channels, 1, in_h, in_w,
                    kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w))
         return 0;
-    if (forward_takes_implicit(batch, in_channels, in_h, in_w, kernel_h, kernel_w, stride_h,
-                               stride_w, pad_h, pad_w))
-        return 0;
-    return col_round_bytes(batch, in_channels, in_h, in_w, kernel_h, kernel_w, stride_h, stride_w,
-                     pad_h, pad_w);
+    return forward_workspace(batch, in_channels, in_h, in_w, kernel_h, kernel_w, stride_h, stride_w,
+                             pad_h, pad_w);
 }
 
 int cdx_conv2d_forward_implicit_f32(const float* input, const float* weight, const float* bias,
@@ -405,6 +447,15 @@ int cdx_conv2d_forward_implicit_f32(const float* input, const float* weight, con
     if (!cdx::conv_fwd_implicit_ok(batch, in_channels, in_h, in_w, kernel_h, kernel_w, stride_h,
                                    stride_w, pad_h, pad_w))
         return set_error(CDX_ERR_UNSUPPORTED, std::string(fn) + ": geometry beyond 32-bit indices");
+    if (cdx::conv_direct_ok(batch, in_channels, out_channels, in_h, in_w, kernel_h, kernel_w,
+                            stride_h, stride_w, pad_h, pad_w) &&
+        cdx::conv_direct_pays(batch * OH * OW, out_channels, in_channels * kernel_h * kernel_w,
+                              cdx::conv_rowwin_ok(batch, in_channels, out_channels, in_h, in_w,
+                                                  kernel_h, kernel_w, stride_h, stride_w, pad_h,
+                                                  pad_w)))
+        return cdx::launch_conv_direct_f32(input, weight, bias, output, batch, in_channels,
+                                           out_channels, in_h, in_w, kernel_h, kernel_w, stride_h,
+                                           stride_w, pad_h, pad_w, stream);
     return cdx::launch_conv_fwd_implicit_f32(input, weight, bias, output, batch, in_channels,
                                              out_channels, in_h, in_w, kernel_h, kernel_w,
                                              stride_h, stride_w, pad_h, pad_w, stream);
@@ -480,12 +531,28 @@ int cdx_conv2d_forward_f32(const float* input, const float* weight, const float*
                            int64_t kernel_w, int64_t stride_h, int64_t stride_w, int64_t pad_h,
                            int64_t pad_w, int precision, void* workspace,
                            size_t workspace_bytes, hipStream_t stream) {
-    if (!check_conv("cdx_conv2d_forward_f32", batch, in_channels, out_channels, in_h, in_w,
-                    kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w) &&
-        forward_takes_implicit(batch, in_channels, in_h, in_w, kernel_h, kernel_w, stride_h,
-                               stride_w, pad_h, pad_w)) {
-        if (!valid_precision(precision))
-            return set_error(CDX_ERR_INVALID_ARG, "cdx_conv2d_forward_f32: bad precision");
+    const char* fn = "cdx_conv2d_forward_f32";
+    int st = check_conv(fn, batch, in_channels, out_channels, in_h, in_w, kernel_h, kernel_w,
+                        stride_h, stride_w, pad_h, pad_w);
+    if (st) return st;
+    if (!valid_precision(precision))
+        return set_error(CDX_ERR_INVALID_ARG, std::string(fn) + ": bad precision");
+    const bool product = conv_is_product(batch, in_channels, out_channels, kernel_h, kernel_w,
+                                         stride_h, stride_w, pad_h, pad_w);
+    if (product || forward_takes_implicit(batch, in_channels, in_h, in_w, kernel_h, kernel_w,
+                                          stride_h, stride_w, pad_h, pad_w)) {
+        const int64_t S = conv_out(in_h, kernel_h, stride_h, pad_h) *
+                          conv_out(in_w, kernel_w, stride_w, pad_w);
+        if (batch == 0 || out_channels == 0 || S == 0) return CDX_OK;
+        if (!output || !weight || !input)
+            return set_error(CDX_ERR_INVALID_ARG, std::string(fn) + ": NULL pointer");
+        if (workspace &&
+            workspace_bytes < forward_workspace(batch, in_channels, in_h, in_w, kernel_h, kernel_w,
+                                                stride_h, stride_w, pad_h, pad_w))
+            return set_error(CDX_ERR_WORKSPACE, std::string(fn) + ": workspace too small");
+        if (product)
+            return conv_product(weight, out_channels, in_channels, input, bias, output, batch, S,
+                                false, stream);
         return cdx_conv2d_forward_implicit_f32(input, weight, bias, output, batch, in_channels,
                                                out_channels, in_h, in_w, kernel_h, kernel_w,
                                                stride_h, stride_w, pad_h, pad_w, stream);
@@ -493,6 +560,18 @@ int cdx_conv2d_forward_f32(const float* input, const float* weight, const float*
     return conv_forward_im2col(input, weight, bias, output, batch, in_channels, out_channels,
                                in_h, in_w, kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w,
                                precision, workspace, workspace_bytes, stream, false);
+}
+
+// A 3x3 stride-1 layer that Winograd's three launches (transforms and 36
+// products, each a pass over memory) do not pay for: up to 1 GFLOP of direct
+// products, with k long enough to split (forward, Winograd against direct, us:
+// 1 x 16 -> 128, 7^2 15 / 8; 2 x 62 -> 23, 31^2 18 / 10; 8 x 24 -> 50, 60^2 28
+// / 22; 4 x 128 -> 128, 28^2 25 / 23; 1.85 GFLOP, 8 x 64 -> 64, 56^2 29 / 39).
+int cdx_conv2d_3x3_is_small(int64_t batch, int64_t in_channels, int64_t out_channels,
+                            int64_t out_h, int64_t out_w) {
+    const long double flops = 18.0L * batch * in_channels * out_channels * out_h * out_w;
+    return batch > 0 && out_h > 0 && out_w > 0 && out_channels > 0 && in_channels * 9 >= 128 &&
+           flops <= 1e9L;
 }
 
 size_t cdx_conv2d_winograd_workspace_size(int64_t batch, int64_t in_channels,
@@ -746,6 +825,17 @@ int cdx_conv2d_backward_data_f32(const float* grad_output, const float* weight, 
     st = ws.acquire(workspace, workspace_bytes, need, stream, fn);
     if (st) return st;
     if (bwd_data_rowwin(batch, in_channels, out_channels, in_h, in_w, kernel_h, kernel_w,
+                        stride_h, stride_w, pad_h, pad_w) &&
+        conv_is_product(batch, in_channels, out_channels, kernel_h, kernel_w, stride_h, stride_w,
+                        pad_h, pad_w)) {
+        float* wt = static_cast<float*>(ws.ptr);
+        st = cdx::launch_flip_filter_f32(weight, wt, out_channels, in_channels, 1, stream);
+        if (!st)
+            st = conv_product(wt, in_channels, out_channels, grad_output, nullptr, grad_input, batch,
+                              in_h * in_w, true, stream);
+        return ws.release(st);
+    }
+    if (bwd_data_rowwin(batch, in_channels, out_channels, in_h, in_w, kernel_h, kernel_w,
                         stride_h, stride_w, pad_h, pad_w)) {
         // stride 1: grad_input = conv(grad_out, flipped filter, padding KH-1-PH, KW-1-PW)
         // through the row-window implicit kernel (FP32 products in every
@@ -756,7 +846,15 @@ int cdx_conv2d_backward_data_f32(const float* grad_output, const float* weight, 
         float* wf = static_cast<float*>(ws.ptr);
         st = cdx::launch_flip_filter_f32(weight, wf, out_channels, in_channels,
                                          kernel_h * kernel_w, stream);
-        if (!st)
+        if (!st && cdx::conv_direct_pays(batch * in_h * in_w, in_channels,
+                                         out_channels * kernel_h * kernel_w, true) &&
+            cdx::conv_direct_ok(batch, out_channels, in_channels, z.OH, z.OW, kernel_h, kernel_w, 1,
+                                1, kernel_h - 1 - pad_h, kernel_w - 1 - pad_w))
+            st = cdx::launch_conv_direct_f32(grad_output, wf, nullptr, grad_input, batch,
+                                             out_channels, in_channels, z.OH, z.OW, kernel_h,
+                                             kernel_w, 1, 1, kernel_h - 1 - pad_h,
+                                             kernel_w - 1 - pad_w, stream);
+        else if (!st)
             st = cdx::launch_conv_rowwin_f32(grad_output, wf, nullptr, grad_input, batch,
                                              out_channels, in_channels, z.OH, z.OW, kernel_h,
                                              kernel_w, 1, 1, kernel_h - 1 - pad_h,

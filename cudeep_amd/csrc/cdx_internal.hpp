@@ -237,6 +237,15 @@ int launch_conv_wgrad_f32(const float* dy, const float* x, float* dw, float* ws,
                           int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH, int64_t KW,
                           int64_t SH, int64_t SW, int64_t PH, int64_t PW, hipStream_t stream);
 
+// The same without LDS staging (conv_wgrad_direct.hip): out is
+// [slices][OC][IC*KH*KW] partials, or dw itself for one slice.
+bool conv_wgrad_direct_ok(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH,
+                          int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW);
+int launch_conv_wgrad_direct_f32(const float* dy, const float* x, float* out, int slices,
+                                 int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
+                                 int64_t KH, int64_t KW, int64_t SH, int64_t SW, int64_t PH,
+                                 int64_t PW, hipStream_t stream);
+
 // Conv forward as an implicit GEMM (FP32 MFMA, operands gathered from the
 // NCHW input while staging k-tiles; no column buffer), with bias; output
 // NCHW.  conv_fwd_implicit_ok() gives the geometries it takes (32-bit
@@ -257,6 +266,17 @@ int launch_conv_rowwin_f32(const float* x, const float* w, const float* bias, fl
                            int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
                            int64_t KH, int64_t KW, int64_t SH, int64_t SW, int64_t PH,
                            int64_t PW, bool two_level, hipStream_t stream);
+
+// The same product with every wave gathering its operands itself, k split over
+// the waves where the layer is small (conv_direct.hip); k summed in two levels.
+bool conv_direct_ok(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH,
+                    int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW);
+// N: batch * OH * OW; rowwin: conv_rowwin_ok()
+bool conv_direct_pays(int64_t N, int64_t OC, int64_t Kc, bool rowwin);
+int launch_conv_direct_f32(const float* x, const float* w, const float* bias, float* y,
+                           int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
+                           int64_t KH, int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW,
+                           hipStream_t stream);
 
 int launch_col2im_f32(const float* col, float* grad_in, int64_t batch, int64_t IC,
                       int64_t IH, int64_t IW, int64_t KH, int64_t KW,

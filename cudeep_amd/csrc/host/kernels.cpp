@@ -212,9 +212,10 @@ void launch_conv2d_forward_kernel<float>(const float* input, const float* weight
     const ConvAlgorithm algo = get_conv_algorithm();
     if (algo == ConvAlgorithm::Winograd && !wino_ok)
         throw std::runtime_error("conv2d: Winograd needs a 3x3 kernel with stride 1");
-    const bool wino = algo == ConvAlgorithm::Winograd ||
-                      (algo == ConvAlgorithm::Auto && wino_ok && OH * OW >= 16);
-    if (algo == ConvAlgorithm::Implicit) {
+    const bool autow = algo == ConvAlgorithm::Auto && wino_ok && OH * OW >= 16;
+    const bool small = autow && cdx_conv2d_3x3_is_small(batch, IC, OC, OH, OW);
+    const bool wino = algo == ConvAlgorithm::Winograd || (autow && !small);
+    if (algo == ConvAlgorithm::Implicit || small) {
         CUDEEP_CHECK_CDX(cdx_conv2d_forward_implicit_f32(input, weight, bias, output, batch, IC,
                                                          OC, IH, IW, KH, KW, SH, SW, PH, PW,
                                                          stream));
@@ -260,7 +261,7 @@ void launch_conv2d_backward_data_kernel<float>(const float* grad_output, const f
             "conv2d backward: Winograd needs a 3x3 kernel with stride 1 and padding <= 2");
     const bool wino = algo == ConvAlgorithm::Winograd ||
                       (algo == ConvAlgorithm::Auto && wino_ok && (int64_t)IH * IW >= 16 &&
-                       prec != CDX_PREC_FP32);
+                       prec != CDX_PREC_FP32 && !cdx_conv2d_3x3_is_small(batch, OC, IC, IH, IW));
     if (wino) {
         Workspace ws(cdx_conv2d_backward_data_winograd_workspace_size(batch, IC, OC, IH, IW, PH,
                                                                       PW),

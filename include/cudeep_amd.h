@@ -216,7 +216,7 @@ int cdx_im2col_f32(const float* input, float* col,
 /* Bytes of workspace cdx_conv2d_forward_f32 needs: the im2col buffer of one
  * round of images (the whole batch while its buffer stays within 128 MiB,
  * else rounds below that sized for whole waves of GEMM tiles), or 0 for
- * layers it sends to the implicit GEMM (see below). */
+ * layers beyond 4 MiB of columns that form none (see below). */
 size_t cdx_conv2d_forward_workspace_size(
     int64_t batch, int64_t in_channels, int64_t in_h, int64_t in_w,
     int64_t kernel_h, int64_t kernel_w, int64_t stride_h, int64_t stride_w,
@@ -225,10 +225,11 @@ size_t cdx_conv2d_forward_workspace_size(
 /* NCHW conv forward: im2col -> one GEMM weight[OC,K_col] * col -> NCHW
  * output with the bias added in the GEMM epilogue (no transpose pass), per
  * round of images (same sums as one pass over the batch).
- * Layers whose column buffer would exceed 4 MiB, other than 3x3 stride-1
- * layers with >= 16 output pixels per image, run the implicit GEMM of
- * cdx_conv2d_forward_implicit_f32 instead (no workspace), as the reference
- * dispatches them to its implicit kernel (conv_kernel.cu:263-275).
+ * Layers other than 3x3 stride-1 ones run the implicit GEMM
+ * of cdx_conv2d_forward_implicit_f32 instead (forming no columns;
+ * the reference sends those beyond 4 MiB of columns to its implicit kernel,
+ * conv_kernel.cu:263-275), and 1x1 stride-1 unpadded ones one product per image
+ * of the tensors as they lie; both with FP32 products in every precision.
  * Replaces cudeep::kernels::launch_conv2d_forward_kernel<float>
  * (include/cudeep/kernels/conv.cuh:8-16, src/kernels/conv_kernel.cu:225-335).
  * bias may be NULL.  precision is CDX_PREC_*.  workspace may be NULL. */
@@ -244,7 +245,8 @@ int cdx_conv2d_forward_f32(const float* input, const float* weight,
 
 /* NCHW conv forward as an implicit GEMM: each tile's input window is staged
  * in LDS once per chunk of input channels (the taps become LDS offsets), or,
- * where that window does not fit, gathered per k-tile; FP32 products, fp32
+ * for small layers and where that window does not fit, every wave gathers its
+ * own operands; FP32 products, fp32
  * accumulation, bias added, no column buffer and no workspace.  Replaces
  * implicit_gemm_conv2d_kernel (src/kernels/conv_kernel.cu:172-215).
  * Geometries needing 64-bit pixel or in-image indices return
@@ -256,6 +258,13 @@ int cdx_conv2d_forward_implicit_f32(const float* input, const float* weight,
                                     int64_t kernel_h, int64_t kernel_w,
                                     int64_t stride_h, int64_t stride_w,
                                     int64_t pad_h, int64_t pad_w, hipStream_t stream);
+
+/* 1 where a 3x3 stride-1 convolution is small enough that the implicit GEMM
+ * (forward; for backward data cdx_conv2d_backward_data_f32, asked with the
+ * transposed layer's channels and grad_input's size) beats Winograd's three
+ * passes, else 0. */
+int cdx_conv2d_3x3_is_small(int64_t batch, int64_t in_channels, int64_t out_channels,
+                            int64_t out_h, int64_t out_w);
 
 /* Bytes of workspace cdx_conv2d_forward_winograd_f32 needs:
  * 36 * (OC*IC + IC*T + OC*T) floats, T = batch * ceil(OH/4) * ceil(OW/4). */
