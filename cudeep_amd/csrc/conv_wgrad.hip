@@ -797,6 +797,25 @@ void launch_rows(const RwPlan& r, dim3 grid, dim3 b16, dim3 b64, const RwArgs& p
 
 }  // namespace
 
+// Where the kernel without LDS staging (conv_wgrad_direct.hip) is the faster
+// one, on the same slices: small layers, whose staged tiles are too few to
+// cover their own latencies; output rows that fill less than half of a row
+// segment; channel counts that pad a 64-channel tile; 1x1 layers, whose filter
+// elements it reads 16 bytes at a time.  Staged / direct, us:
+//   rows kernel   1 x 16 -> 128, 7^2      21 / 8     4 x 64 -> 64, 28^2 (0.23 GFLOP)   19 / 15
+//                 16 x 128 -> 128, 14^2   42 / 33    32 x 256 -> 256, 14^2            207 / 148
+//                 8 x 24 -> 50, 60^2 (0.62 GFLOP) 30 / 34     32 x 64 -> 64, 56^2      86 / 130
+//   gather kernel 6 x 56 -> 46, 31^2, 3x3 s2      29 / 13     8 x 64 -> 128, 56^2, s2  33 / 29
+//                 20 x 128 -> 168, 28^2, 7x7 s2  200 / 161    16 x 16 -> 32, 112^2, 5x5 199 / 129
+//                 1 x 76 -> 128, 60^2, 7x7        63 / 67     16 x 3 -> 64, 224^2, 7x7 s2 84 / 88
+//   1x1           16 x 256 -> 64, 56^2            49 / 43     8 x 128 -> 64, 31^2       31 / 14
+static bool direct_pays(const WgGeom& g) {
+    const long double flops = 2.0L * g.B * g.S() * g.OC * g.Kc();
+    if (g.KH == 1 && g.KW == 1 && g.SH == 1 && g.SW == 1 && g.PH == 0 && g.PW == 0) return true;
+    if (rows_applies(g)) return flops <= 0.5e9L || g.OW <= 16;
+    return flops <= 1e9L || ceil_div(g.OC, WG_BM) * WG_BM * 100 >= g.OC * 112;
+}
+
 bool conv_wgrad_implicit_ok(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
                             int64_t KH, int64_t KW, int64_t SH, int64_t SW, int64_t PH,
                             int64_t PW) {
@@ -821,6 +840,15 @@ int launch_conv_wgrad_f32(const float* dy, const float* x, float* dw, float* ws,
                           int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH, int64_t KW,
                           int64_t SH, int64_t SW, int64_t PH, int64_t PW, hipStream_t stream) {
     const WgGeom g = make_geom(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW);
+    if (direct_pays(g) && conv_wgrad_direct_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)) {
+        const int splits = rows_applies(g) ? rw_plan(g).splits : splits_for(g);
+        int st = launch_conv_wgrad_direct_f32(dy, x, splits > 1 ? ws : dw, splits, batch, IC, OC, IH,
+                                              IW, KH, KW, SH, SW, PH, PW, stream);
+        if (st || splits == 1) return st;
+        GemmArgs red{CDX_OP_N, CDX_OP_N, OC, g.Kc(), 0, nullptr, 1, nullptr, 1, dw, g.Kc(), 0, 0,
+                     nullptr, CDX_BIAS_NONE, CDX_EPI_NONE};
+        return launch_splitk_reduce(ws, splits, red, stream);
+    }
     if (rows_applies(g)) {
         const RwPlan r = rw_plan(g);
         RwArgs p;
