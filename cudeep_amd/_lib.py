@@ -127,4 +127,6 @@ def check(code: int) -> None:
 
 def call(name: str, *args) -> None:
     """Call an int-returning entry point and raise CdxError on failure."""
-    check(getattr(lib(), name)(*args))
+    code = getattr(_lib or lib(), name)(*args)
+    if code != CDX_OK:
+        check(code)

@@ -13,8 +13,17 @@ import ctypes
 from . import _lib as L
 
 
-def _stream():
-    return ctypes_stream(torch.cuda.current_stream())
+# The current stream of the current device as an integer.  Asked for directly:
+# torch.cuda.current_stream() builds a Stream object through several Python
+# layers, 2.9 us of an 8 to 13 us call, against 0.2.
+_current_device = torch._C._cuda_getDevice if hasattr(torch._C, "_cuda_getDevice") else None
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
+def _stream() -> int:
+    if _current_device is None or _raw_stream is None:
+        return ctypes_stream(torch.cuda.current_stream())
+    return _raw_stream(_current_device())
 
 
 def ctypes_stream(s) -> int:
@@ -34,9 +43,11 @@ def _ld(t: torch.Tensor, name: str) -> int:
     """Leading dimension of a row-major 2-D view (unit column stride)."""
     if t.dim() != 2:
         raise ValueError(f"{name} must be 2-D")
-    if t.stride(1) != 1 and t.size(1) > 1:
+    ld, step = t.stride()
+    cols = t.shape[1]
+    if step != 1 and cols > 1:
         raise ValueError(f"{name} must have unit column stride")
-    return max(t.stride(0), t.size(1), 1)
+    return ld if ld >= cols and ld >= 1 else max(cols, 1)
 
 
 def _scratch(workspace, nbytes, device):
