@@ -131,6 +131,9 @@ int launch_gemm_parts(const GemmArgs& g, hipStream_t stream);
 bool gemm_direct_ok(const GemmArgs& g);
 bool gemm_direct_for_tf32(const GemmArgs& g);
 int launch_gemm_direct(const GemmArgs& g, hipStream_t stream);
+// The same for 16-bit operands (gemm_direct16.hip; plain output map, no batch).
+bool gemm_direct16_ok(const GemmArgs& g);
+int launch_gemm_direct16(const GemmArgs& g, bool bf16, hipStream_t stream);
 int launch_dgemm(int opA, int opB, int64_t M, int64_t N, int64_t K,
                  const double* A, int64_t lda, const double* B, int64_t ldb,
                  double* C, int64_t ldc, hipStream_t stream);

@@ -114,6 +114,7 @@ int launch_gemm_bf16x3(const GemmArgs& g, int terms, hipStream_t stream) {
 }
 
 int launch_gemm_16(const GemmArgs& g, int in_dtype, hipStream_t stream) {
+    if (gemm_direct16_ok(g)) return launch_gemm_direct16(g, in_dtype == CDX_DTYPE_BF16, stream);
     return in_dtype == CDX_DTYPE_BF16 ? dispatch16<kInBF16>(g, stream) : dispatch16<kInF16>(g, stream);
 }
 
