@@ -174,16 +174,12 @@ inline size_t splitk_bytes(const GemmArgs& g, int64_t tiles, int bk, int64_t min
     return splits > 1 ? (size_t)splits * (size_t)g.M * (size_t)g.N * sizeof(float) : 0;
 }
 
-// Runs a GEMM whose tile grid is `tiles` through split-K when the policy
-// asks for it: takes the partials from g.ws (or allocates them stream-
-// ordered), calls launch(kparams-adjusted GemmArgs, splits, k_chunk) and
-// reduces.
+// Runs a GEMM as `splits` slices of k_chunk k: takes the partials from g.ws (or
+// allocates them stream-ordered), calls launch(kparams-adjusted GemmArgs,
+// splits, k_chunk) and reduces.  One slice: launch(g, 1, K).
 template <class LaunchFn>
-int with_splitk(const GemmArgs& g, int64_t tiles, int bk, hipStream_t stream, LaunchFn launch,
-                int64_t min_k = 256) {
-    int64_t k_chunk;
-    const int splits = g.batch > 1 ? (k_chunk = g.K, 1)
-                                   : choose_splitk(tiles, g.K, bk, &k_chunk, min_k);
+int with_slices(const GemmArgs& g, int splits, int64_t k_chunk, hipStream_t stream,
+                LaunchFn launch) {
     if (splits == 1) return launch(g, 1, g.K);
     float* part = static_cast<float*>(g.ws);
     const size_t bytes = (size_t)splits * (size_t)g.M * (size_t)g.N * sizeof(float);
@@ -205,6 +201,16 @@ int with_splitk(const GemmArgs& g, int64_t tiles, int bk, hipStream_t stream, La
         if (!st) st = st2;
     }
     return st;
+}
+
+// The same with the slices the policy chooses for a tile grid of `tiles`.
+template <class LaunchFn>
+int with_splitk(const GemmArgs& g, int64_t tiles, int bk, hipStream_t stream, LaunchFn launch,
+                int64_t min_k = 256) {
+    int64_t k_chunk;
+    const int splits = g.batch > 1 ? (k_chunk = g.K, 1)
+                                   : choose_splitk(tiles, g.K, bk, &k_chunk, min_k);
+    return with_slices(g, splits, k_chunk, stream, launch);
 }
 
 int launch_im2col_f32(const float* in, float* col, int64_t batch, int64_t IC,

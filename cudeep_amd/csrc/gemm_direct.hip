@@ -234,7 +234,8 @@ bool gemm_direct_ok(const GemmArgs& g) {
 // element (1021 x 765 x 1533 NT 32.5 against 63.7, 1336 x 576 x 381 TN 12.7
 // against 18.5; with 16-byte rows 2000 x 700 x 500 24.4 against 21.3).
 bool gemm_direct_for_tf32(const GemmArgs& g) {
-    if (g.n_split > 0 || !gemm_direct_ok(g)) return false;
+    // (wide 64-row products keep the split kernel's own k-slices)
+    if (g.n_split > 0 || (g.M <= 64 && g.N >= 4096) || !gemm_direct_ok(g)) return false;
     const int64_t t32 = tiles_of(g, 32);
     const KParams kp = f32::kparams_of(g, g.K);
     return t32 <= 256 || (t32 <= 1024 && !(kp.vec_a && kp.vec_b));

@@ -14,7 +14,12 @@ size_t gemm_f32_workspace(const GemmArgs& g) {
 
 int launch_gemm_f32(const GemmArgs& g, hipStream_t stream) {
     if (narrow_kind(g)) return launch_gemm_narrow(g, stream);
-    if (gemm_parts_ok(g)) return launch_gemm_parts(g, stream);
+    // a caller's workspace is held to what the tiled route needs; one too small
+    // for the three-part kernel's slices leaves the product to the others
+    if (g.ws && g.ws_bytes < gemm_f32_tiled_workspace(g))
+        return set_error(CDX_ERR_WORKSPACE, "gemm: workspace too small");
+    if (gemm_parts_ok(g) && !(g.ws && g.ws_bytes < gemm_parts_workspace(g)))
+        return launch_gemm_parts(g, stream);
     if (gemm_direct_ok(g)) return launch_gemm_direct(g, stream);
     return launch_gemm_f32_tiled(g, stream);
 }

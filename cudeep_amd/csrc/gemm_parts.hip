@@ -424,24 +424,49 @@ int64_t own_tiles(const GemmArgs& g) {
     return ceil_div(g.M, PTile::BM) * ceil_div(nb, PTile::BN);
 }
 
-// The tile count that the k-slices are chosen for: that of the tiled kernel's
-// 128 x 64 slice tiles where it would split too, so that both routes take the
-// same slices (and ask for the same workspace).
-int64_t slice_tiles(const GemmArgs& g) {
-    const int64_t nb = g.ones_col >= 0 ? g.ones_col : g.N;
-    const int64_t t = ceil_div(g.M, 128) * ceil_div(nb, 64);
-    return splitk_applies(t, g.K) ? t : own_tiles(g);
+// k-slices of a product that does not fill the GPU with its tiles, where K is
+// long enough to split (splitk_applies, on these tiles or the tiled kernel's
+// slices): the count whose rounds of one workgroup per CU, each its k-tiles
+// and about four more for filling the pipeline and the epilogue, plus the pass
+// over the partials, are shortest.  256 x 785 x 8192, 14 tiles: 18 slices, one
+// round: 38 us with the reduction against 47 in the 29 slices, two rounds, of the
+// tiled kernel's policy (made for workgroups of which two or three share a CU).
+struct Slices {
+    int n;
+    int64_t chunk;
+};
+
+Slices slices_of(const GemmArgs& g) {
+    const int64_t nb = g.ones_col >= 0 ? g.ones_col : g.N, t = own_tiles(g);
+    if (g.batch > 1 || !(splitk_applies(t, g.K) ||
+                         splitk_applies(ceil_div(g.M, 128) * ceil_div(nb, 64), g.K)))
+        return {1, g.K};
+    const int64_t nk = ceil_div(g.K, PBK);
+    Slices best{1, g.K};
+    double least = 0.0;
+    for (int64_t s = 1; s <= nk / 8 && s <= 256; ++s) {
+        const int64_t per = ceil_div(nk, s), n = ceil_div(nk, per);
+        // (a k-tile takes about 0.75 us; partials move at about 4 TB/s)
+        const double cost = (double)ceil_div(t * n, 256) * (double)(per + 4) +
+                            (n > 1 ? 5.0 + (double)n * (double)(g.M * nb) * 1.3e-6 : 0.0);
+        if (s == 1 || cost < least) {
+            least = cost;
+            best = {(int)n, n > 1 ? per * PBK : g.K};
+        }
+    }
+    return best;
 }
 
 }  // namespace
 
 // Which products: those with a 128 x 128 tile for nearly every CU (2048^3 92
 // against 131 us on the fp32 matrix path, 8192 x 784 x 256 33 against 36, 5079
-// x 896 x 920 NT 88 against 93), or with k-slices of such tiles (256 x 785 x
-// 8192 TN 47 against 49; 2539 x 704 x 2624 NT 88 against 124).  With fewer
-// tiles and a short K the smaller fp32 tiles win: 8192 x 256 x 784 NT (128
-// tiles) 38 against 32, 1536^3 69 against 67, 1024^3 48 against 26.  Tiles
-// may be padded by up to 40 %.  Operand panels are addressed with 32-bit
+// x 896 x 920 NT 88 against 93), or with enough k-slices of such tiles (256 x
+// 785 x 8192 TN 38 against 49; 2539 x 704 x 2624 NT 76 against 124; 512 x 1024
+// x 8192 TN 67 against 181; 64 workgroups, 256 x 257 x 4096 TN, 24 against 22).
+// With fewer tiles and a short K the smaller fp32 tiles win: 8192 x 256 x 784
+// NT (128 tiles) 38 against 32, 1536^3 69 against 67, 1024^3 48 against 26.
+// Tiles may be padded by up to 40 %.  Operand panels are addressed with 32-bit
 // offsets.
 bool gemm_parts_ok(const GemmArgs& g) {
     const int64_t nb = g.ones_col >= 0 ? g.ones_col : g.N, lim = int64_t(1) << 22;
@@ -450,16 +475,22 @@ bool gemm_parts_ok(const GemmArgs& g) {
         return false;
     const int64_t tiles = own_tiles(g);
     if (tiles > INT32_MAX / 2 || tiles * (PTile::BM * PTile::BN) > g.M * nb / 5 * 7) return false;
-    return tiles >= 240 || (g.batch == 1 && splitk_applies(tiles, g.K));
+    if (tiles >= 240) return true;
+    const int n = slices_of(g).n;
+    return n > 1 && tiles * n >= 160;
 }
 
-size_t gemm_parts_workspace(const GemmArgs& g) { return splitk_bytes(g, slice_tiles(g), PBK); }
+size_t gemm_parts_workspace(const GemmArgs& g) {
+    const int n = slices_of(g).n;
+    return n > 1 ? (size_t)n * (size_t)g.M * (size_t)g.N * sizeof(float) : 0;
+}
 
 int launch_gemm_parts(const GemmArgs& g0, hipStream_t stream) {
     const int64_t tiles = ceil_div(g0.M, PTile::BM) * ceil_div(g0.N, PTile::BN);
     if (tiles > INT32_MAX) return set_error(CDX_ERR_UNSUPPORTED, "gemm: too many tiles");
     if (g0.batch < 1 || g0.batch > 65535) return set_error(CDX_ERR_UNSUPPORTED, "gemm: batch out of range");
-    return with_splitk(g0, slice_tiles(g0), PBK, stream,
+    const Slices sl = slices_of(g0);
+    return with_slices(g0, sl.n, sl.chunk, stream,
                        [&](const GemmArgs& g, int splits, int64_t k_chunk) {
         const KParams kp = f32::kparams_of(g, k_chunk);
         const dim3 grid((unsigned)tiles, (unsigned)splits, (unsigned)g.batch), block(PTile::NT);

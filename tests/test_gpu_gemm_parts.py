@@ -95,6 +95,24 @@ def test_slices_with_ones_column(M, N, K, tB):
     assert oracle.rel_fro(host(cs), db64) <= 2 * oracle.rel_fro(oracle.colsum(A), db64) + 2.0 ** -24
 
 
+@pytest.mark.parametrize("M,N,K", [(1000, 1001, 4097), (1029, 1150, 2331)])
+def test_slices_and_workspaces(M, N, K):
+    """Own slices with ragged tiles and k, on a workspace of the queried size and on one too small
+    for them (the product then takes another route, with as good a result)."""
+    import torch
+    rng = np.random.default_rng(M + K)
+    A, B = normal(rng, (M, K)), normal(rng, (N, K))
+    need = ops().gemm_workspace_bytes(M, N, K, transB=True)
+    say("gemm parts workspaces", M, N, K, need)
+    C = ops().gemm(dev(A), dev(B), transB=True)
+    _check(host(C), A, B, False, True, _rows(M))
+    assert need > 0
+    ws = torch.empty(need // 4, device="cuda")
+    assert torch.equal(C, ops().gemm(dev(A), dev(B), transB=True, workspace=ws))
+    _check(host(ops().gemm(dev(A), dev(B), transB=True, workspace=ws[:4])), A, B, False, True,
+           _rows(M))
+
+
 @pytest.mark.parametrize("sa,sb", [(-118, 20), (-118, 100), (60, -70), (20, -118), (-60, -50)])
 def test_scales(sa, sb):
     """Operands scaled by powers of two, out of the range of exact parts on one side or both
