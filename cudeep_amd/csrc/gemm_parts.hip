@@ -23,12 +23,15 @@
 // i.e. for |x| >= 2^-110 (or 0), and finite for |x| below bf16's rounding
 // limit.  An output can lose accuracy only if every |a| of its row (or |b| of
 // its column) is below 2^-110; with the other operand below 2^40 and K <=
-// 2^16 such an output is below 2^-54.  So a workgroup recomputes its tile
-// with the fp32 matrix instruction (f32::gemm_tile, the same arithmetic as
-// gemm_f32.hip) when it staged an |x| >= 2^40 (infinities among them), or
-// some accumulator is NaN, or nonzero and below 2^-54.  On data without such
-// values this costs one v_max3 per two staged elements and three compares
-// per output.
+// 2^16 such an output is below 2^-54; it is zero only if subnormals vanished.
+// So a workgroup recomputes its tile with the fp32 matrix instruction
+// (f32::gemm_tile, the same arithmetic as gemm_f32.hip) when it staged an
+// |x| >= 2^40 (infinities among them), or some accumulator is NaN, or nonzero
+// and below 2^-54, or zero where a subnormal was staged.  On data without such
+// values this costs four VALU operations per two staged elements and four
+// compares per output (8192 x 784 x 256 33.3 us against 32.6 without the search
+// for subnormals, 4096^3 the same; a class compare per element instead 36, and
+// a second pass over the operands of tiles with a zero output 43 with zero rows).
 //
 // Structure (per workgroup, one 128 x 128 output tile, k-tiles of 32): eight
 // waves in two groups of four, one wave of each per SIMD.  Each group owns the
@@ -174,8 +177,10 @@ struct PartLoader {
         }
     }
     // Splits into the three planes at s ([mn][PSTRIDE], `plane` apart);
-    // amax: the largest magnitude seen.
-    __device__ __forceinline__ void store(unsigned short* s, int plane, float& amax, int tid) const {
+    // amax: the largest magnitude seen; least: the smallest but 0, as its bits
+    // without the sign, doubled, less one.
+    __device__ __forceinline__ void store(unsigned short* s, int plane, float& amax,
+                                          uint32_t& least, int tid) const {
 #pragma unroll
         for (int b = 0; b < NV; ++b) {
             int bc, br;
@@ -187,6 +192,11 @@ struct PartLoader {
                 else x = f32x4u{v[b][0][r], v[b][1][r], v[b][2][r], v[b][3][r]};
                 asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(amax) : "v"(x.x), "v"(x.y));
                 asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(amax) : "v"(x.z), "v"(x.w));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t u = (__builtin_bit_cast(uint32_t, x[i]) << 1) - 1u;
+                    least = u < least ? u : least;
+                }
                 uint2 h, m, l;
                 split3(x.x, x.y, h.x, m.x, l.x);
                 split3(x.z, x.w, h.y, m.y, l.y);
@@ -212,7 +222,7 @@ void gemm_parts_kernel(KParams p) {
     constexpr int STAGE = 3 * (A_PLANE + B_PLANE);   // bf16
     using Fallback = CF::Fallback;
     __shared__ __attribute__((aligned(16))) unsigned short lds[2 * STAGE];
-    __shared__ int redo;
+    __shared__ int redo, subnormals, zeros;
     static_assert(2 * STAGE * 2 >= 8 * 8 * 64 * 16, "the hand-over needs 64 KiB");
     static_assert(2 * STAGE * 2 >= f32::Geo<Fallback, OPA, OPB>::LDS_FLOATS * 4, "fallback tile");
 
@@ -266,12 +276,13 @@ void gemm_parts_kernel(KParams p) {
         else if (t < nk) lb.load_tail(pb + t * step_b, p.ldb, krem, tid);
     };
     float amax = 0.0f;
+    uint32_t least = 0xffffffffu;
     auto store = [&](int64_t t) {
         const int kr = t + 1 < nk ? PBK : krem;
         if (edge_a || kr < PBK) la.fix(arem, kr, -1, tid);
-        la.store(sA, A_PLANE, amax, tid);
+        la.store(sA, A_PLANE, amax, least, tid);
         if (edge_b || kr < PBK) lb.fix(brem, kr, one, tid);
-        lb.store(sB, B_PLANE, amax, tid);
+        lb.store(sB, B_PLANE, amax, least, tid);
     };
 
     floatx4 acc[FM][FN];
@@ -334,7 +345,7 @@ void gemm_parts_kernel(KParams p) {
 
     // group g takes the k-tiles g, g + 2, ...; both run the barriers of the
     // longer list, group 1 one slot behind
-    if (threadIdx.x == 0) redo = 0;
+    if (threadIdx.x == 0) redo = subnormals = zeros = 0;
     const int64_t slots = (nk + 1) / 2;
     if (grp < nk) {
         load_a(grp);
@@ -384,7 +395,7 @@ void gemm_parts_kernel(KParams p) {
                 res[i][j] = red[((w * 2 + 1) * 8 + i * FN + j) * 64 + lane] + acc[2 + i][j];
     }
 
-    bool bad = !(amax < kPartsHuge);
+    bool bad = !(amax < kPartsHuge), zero = false;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -393,10 +404,13 @@ void gemm_parts_kernel(KParams p) {
             for (int e = 0; e < 4; ++e) {
                 const float c = __builtin_fabsf(res[i][j][e]);
                 bad |= !(c >= kPartsTiny) && c != 0.0f;   // NaN too
+                zero |= c == 0.0f;
             }
     if (bad) redo = 1;
+    if (zero) zeros = 1;
+    if (least < (2u << 23) - 1u) subnormals = 1;   // (that of 2^-126)
     __syncthreads();
-    if (redo) {   // (uniform) the fp32 matrix path, a smaller tile at a time
+    if (redo || (zeros && subnormals)) {   // (uniform) the fp32 matrix path, a smaller tile at a time
         constexpr int TN = BN / Fallback::BN;
 #pragma unroll 1
         for (int s = 0; s < BM / Fallback::BM * TN; ++s) {

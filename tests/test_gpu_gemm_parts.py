@@ -113,10 +113,11 @@ def test_slices_and_workspaces(M, N, K):
            _rows(M))
 
 
-@pytest.mark.parametrize("sa,sb", [(-118, 20), (-118, 100), (60, -70), (20, -118), (-60, -50)])
+@pytest.mark.parametrize("sa,sb", [(-118, 20), (-118, 100), (60, -70), (20, -118), (-60, -50),
+                                   (-135, 30), (35, -140)])
 def test_scales(sa, sb):
     """Operands scaled by powers of two, out of the range of exact parts on one side or both
-    (and products near the smallest normal number): the same bar."""
+    (and products near the smallest normal number, subnormal operands): the same bar."""
     M, N, K = 2048, 2048, 96
     rng = np.random.default_rng(77)
     A = (normal(rng, (M, K)) * np.float32(2.0) ** sa).astype(np.float32)
@@ -124,6 +125,20 @@ def test_scales(sa, sb):
     say("gemm parts scales", sa, sb)
     C = host(ops().gemm(dev(A), dev(B)))
     _check(C, A, B, False, False, _rows(M))
+
+
+def test_zero_outputs():
+    """Zero rows and columns stay zero; a row of subnormals among them is not taken for one."""
+    M, N, K = 2048, 2050, 70
+    rng = np.random.default_rng(79)
+    A, B = normal(rng, (M, K)), normal(rng, (K, N)) * np.float32(2.0 ** 20)
+    A[3], A[130], B[:, 2049] = 0.0, 0.0, 0.0
+    A[7] = (normal(rng, (K,)).astype(np.float64) * 2.0 ** -139).astype(np.float32)
+    say("gemm parts zero outputs")
+    C = host(ops().gemm(dev(A), dev(B)))
+    assert not C[3].any() and not C[130].any() and not C[:, 2049].any()
+    for r in (2, 7, 131):
+        _check(C, A, B, False, False, [r])
 
 
 def test_mixed_rows():
