@@ -2,8 +2,9 @@
 """Benchmark of the MI355X dense-contraction path (one GPU).
 
 Headline (BASELINE.json metric): FP32 GEMM TFLOP/s at M=N=K=4096 (config
-C2, A, B ~ N(0,1), beta=0) and its fraction of the MI355X FP32 MFMA peak
-(157.3 TFLOP/s).  A "step" is one 4096^3 FP32 GEMM through cdx_sgemm_f32,
+C2, A, B ~ N(0,1), beta=0) and its percentage of the MI355X FP32 MFMA peak
+(157.3 TFLOP/s; more than 100 is possible, since the product runs in exact
+bf16 parts, whose ceiling is the roofline's).  A "step" is one 4096^3 FP32 GEMM through cdx_sgemm_f32,
 with A, B, C resident in HBM.  The same run also reports, under "extra":
 TF32-mode (bf16x3) GEMM at 2048^3 / 4096^3 (C3), the MLP Linear stack (C4)
 and the im2col + GEMM Conv2d (C5).
@@ -36,6 +37,9 @@ sys.path.insert(0, ROOT)
 
 FP32_PEAK_TFLOPS = 157.3      # MI355X dense FP32 MFMA
 BF16_PEAK_TFLOPS = 2516.6     # MI355X dense BF16 MFMA; bf16x3 logical ceiling = /3
+# The headline product runs on the bf16 matrix cores, six products of exact
+# bf16 parts per fp32 product (gemm_parts.hip): its roofline is a sixth of theirs.
+FP32_PARTS_PEAK_TFLOPS = BF16_PEAK_TFLOPS / 6
 HEAD_SETTLE_S = 0.3           # untimed clock-settling launches before the headline
 HBM_PEAK_GBS = 8000.0
 MLP_SETTLE_S = 0.3            # untimed settling launches before each C4 step line
@@ -653,8 +657,9 @@ def main():
         "pct_of_fp32_mfma_peak": round(100 * head["tflops"] / FP32_PEAK_TFLOPS, 2),
         "tf32mode_4096_tflops": (round(extra["tf32mode_4096"]["tflops"], 3)
                                  if "tf32mode_4096" in extra else None),
-        "roofline": {"bound": "mfma", "achieved": round(achieved, 3), "peak": FP32_PEAK_TFLOPS,
-                     "unit": "TFLOP/s", "frac": round(achieved / FP32_PEAK_TFLOPS, 4),
+        "roofline": {"bound": "mfma", "achieved": round(achieved, 3),
+                     "peak": round(FP32_PARTS_PEAK_TFLOPS, 1),
+                     "unit": "TFLOP/s", "frac": round(achieved / FP32_PARTS_PEAK_TFLOPS, 4),
                      "traffic": traffic},
         "cpu_baseline": cpu,
         "extra": extra,

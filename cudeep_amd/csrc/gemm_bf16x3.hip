@@ -79,9 +79,9 @@ int dispatch16(const GemmArgs& g, hipStream_t stream) {
 
 }  // namespace
 
-// Products whose FP32 form runs on 128 x 112 tiles (C4's 8192 x 784 x 256
-// dX) take it in the TF32 modes too: 35.5 against 40.2 us there, with exact
-// products (inside the TF32-mode error bar).
+// Products that 128 x 112 tiles divide well (C4's 8192 x 784 x 256 dX) run in
+// FP32 in the TF32 modes too: 33.3 us in three exact parts (35.5 on 128 x 112
+// fp32 tiles) against 40.2 there (inside the TF32-mode error bar).
 static bool to_f32(const GemmArgs& g, int terms) {
     return narrow_kind(g) || tn_split_to_f32(g, terms) || f32_takes_w112(g) ||
            gemm_direct_for_tf32(g);

@@ -7,6 +7,10 @@
 // the matrix core four k at a time), which is what the relative-Frobenius
 // parity gate compares against.
 //
+// Which products come here is decided in gemm_f32_route.hip: large ones take
+// gemm_parts.hip, small and unaligned ones gemm_direct.hip.  The figures below
+// compare this kernel's configurations with each other.
+//
 // Structure (per workgroup, one BM x BN output tile):
 //   * A and B k-tiles of depth BK are staged global -> VGPR -> LDS with
 //     register double buffering: the loads for tile t+1 are in flight while

@@ -194,7 +194,7 @@ def hgemm(A, B, out=None):
 
 
 def sgemm(A, B, out=None):
-    """C = A @ B, FP32 MFMA (cdx_sgemm_f32); A, B contiguous row-major."""
+    """C = A @ B, FP32 products (cdx_sgemm_f32); A, B contiguous row-major."""
     _need(A, "A")
     _need(B, "B")
     if A.dim() != 2 or B.dim() != 2 or A.shape[1] != B.shape[0]:

@@ -72,7 +72,8 @@ extern "C" {
 #define CDX_BIAS_ROW  1            /* C[m][n] += bias[m]  (conv: per channel) */
 #define CDX_BIAS_COL  2            /* C[m][n] += bias[n]  (Linear)            */
 
-#define CDX_PREC_FP32      0       /* true-FP32 MFMA (v_mfma_f32_16x16x4_f32) */
+#define CDX_PREC_FP32      0       /* fp32 products: fp32 MFMA, or six bf16 MFMAs
+                                      of exact bf16 parts for large ones */
 #define CDX_PREC_TF32MODE  1       /* bf16x3 split MFMA, |rel err| <= 2^-15 per product */
 #define CDX_PREC_TF32MODE4 2       /* bf16x4 split MFMA, |rel err| <= 2^-16 per product;
                                       exact products for operands of <= 16 significant
@@ -93,7 +94,7 @@ const char* cdx_version(void);
 
 /* ---- GEMM ------------------------------------------------------------ */
 
-/* C[M,N] = A[M,K] * B[K,N], FP32 MFMA, C overwritten.
+/* C[M,N] = A[M,K] * B[K,N], FP32 products, C overwritten.
  * Replaces cudeep::kernels::launch_matmul_kernel_fp32<float>
  * (include/cudeep/kernels/matmul.cuh:14-18, src/kernels/matmul_kernel.cu:1851-1863). */
 int cdx_sgemm_f32(const float* A, const float* B, float* C,
