@@ -1323,3 +1323,15 @@ int cdx_sum(const void* x, void* out, int64_t n, int dtype, void* workspace,
 }
 
 }  // extern "C"
+
+// Internal: the kernel that a call with these arguments runs, operands 16-byte
+// aligned, no caller workspace.  `in` is CDX_PREC_* (fp32 operands) or 16 +
+// CDX_DTYPE_* (16-bit ones).
+extern "C" const char* cdxi_gemm_kernel(int in, int opA, int opB, int64_t M, int64_t N, int64_t K,
+                                        int64_t lda, int64_t ldb) {
+    const cdx::GemmArgs g{opA, opB, M, N, K, nullptr, lda, nullptr, ldb, nullptr, N, 0, 0,
+                          nullptr, CDX_BIAS_NONE, CDX_EPI_NONE};
+    if (in >= 16) return cdx::gemm_16_kernel_name(g);
+    if (in == CDX_PREC_FP32) return cdx::gemm_f32_kernel_name(g);
+    return cdx::gemm_bf16x3_kernel_name(g, in == CDX_PREC_TF32MODE4 ? 4 : 3);
+}

@@ -134,6 +134,11 @@ int launch_gemm_direct(const GemmArgs& g, hipStream_t stream);
 // The same for 16-bit operands (gemm_direct16.hip; plain output map, no batch).
 bool gemm_direct16_ok(const GemmArgs& g);
 int launch_gemm_direct16(const GemmArgs& g, bool bf16, hipStream_t stream);
+// Names of the kernels that the launchers above would run (for tests that aim
+// at one of them).
+const char* gemm_f32_kernel_name(const GemmArgs& g);
+const char* gemm_bf16x3_kernel_name(const GemmArgs& g, int terms);
+const char* gemm_16_kernel_name(const GemmArgs& g);
 int launch_dgemm(int opA, int opB, int64_t M, int64_t N, int64_t K,
                  const double* A, int64_t lda, const double* B, int64_t ldb,
                  double* C, int64_t ldc, hipStream_t stream);

@@ -113,6 +113,12 @@ int launch_gemm_bf16x3(const GemmArgs& g, int terms, hipStream_t stream) {
     return terms == 4 ? dispatch<4>(g, stream) : dispatch<3>(g, stream);
 }
 
+const char* gemm_bf16x3_kernel_name(const GemmArgs& g, int terms) {
+    return to_f32(g, terms) ? gemm_f32_kernel_name(g) : "split";
+}
+
+const char* gemm_16_kernel_name(const GemmArgs& g) { return gemm_direct16_ok(g) ? "direct" : "tiled"; }
+
 int launch_gemm_16(const GemmArgs& g, int in_dtype, hipStream_t stream) {
     if (gemm_direct16_ok(g)) return launch_gemm_direct16(g, in_dtype == CDX_DTYPE_BF16, stream);
     return in_dtype == CDX_DTYPE_BF16 ? dispatch16<kInBF16>(g, stream) : dispatch16<kInF16>(g, stream);

@@ -172,6 +172,14 @@ int64_t tiles_of(const GemmArgs& g, int64_t side) { return ceil_div(g.M, side) *
 //   1151 x 102 x 2320 NN 70.8 / 15.6 / 11.5    224 x 704 x 2256 NN  34.6 / 14.8 / 14.5
 //   512^3 NT              6.5 /  8.7 /  5.6    1000 x 500 x 300 TT  10.6 /  7.3 /  6.0
 //   640 x 640 x 1280 TN  21.0 / 23.7 / 10.3    768^3 NT              8.2 / 16.6 / 12.1
+// A wave sums a quarter of K in one accumulator, the tiled kernels' k-slices
+// 1024 k and more each: where those slice, K ends at 4096, beyond which this
+// kernel is the less exact one and soon the slower one too.  Tiled / this, us
+// and relative error against fp64 (bf16, N(0, 1)):
+//   256 x 256 x 4096 NN   19.9 / 12.0   1.9e-7 / 1.9e-7
+//   256 x 256 x 8192 NN   20.6 / 37.2   1.9e-7 / 2.7e-7
+//   256 x 784 x 8192 NN   32.4 / 44.0   1.9e-7 / 2.7e-7
+//   64 x 64 x 65536 NT    20.0 / 112.7  2.4e-7 / 8.5e-7
 bool gemm_direct16_ok(const GemmArgs& g) {
     const int64_t lim = int64_t(1) << 22;
     if (g.n_split > 0 || g.batch != 1 || g.M < 1 || g.N < 1 || g.K < 1 || g.K > INT32_MAX / 2 ||
@@ -182,6 +190,7 @@ bool gemm_direct16_ok(const GemmArgs& g) {
     if (g.opB == CDX_OP_T && ((uintptr_t)g.B % 4 != 0 || g.ldb % 2 != 0)) return false;
     const bool whole = g.M % 64 == 0 && g.N % 64 == 0 && g.K % 64 == 0 && g.lda % 8 == 0 &&
                        g.ldb % 8 == 0 && (uintptr_t)g.A % 16 == 0 && (uintptr_t)g.B % 16 == 0;
+    if (g.K > 4096 && splitk_applies(tiles_of(g, 64), g.K)) return false;
     return tiles_of(g, 32) <= (whole ? 320 : 768);
 }
 
