@@ -165,12 +165,14 @@ int64_t tiles_of(const GemmArgs& g, int64_t side) { return ceil_div(g.M, side) *
 
 }  // namespace
 
-// Up to 320 tiles of 32 x 32, or 768 where the tiled kernels would load element
-// by element; tiles of 16 x 16 up to 400 of them.  Tiled / 16 x 16 / 32 x 32, us:
+// Up to 256 tiles of 32 x 32 (A transposed, B not: 320), or 768 where the tiled
+// kernels would load element by element; tiles of 16 x 16 up to 400 of them.
+// Tiled / 16 x 16 / 32 x 32, us:
 //   256^3 NT              4.9 /  3.2 /  4.1    100 x 100 x 3000 TN  42.4 /  9.2 / 13.3
 //   300^3 NT             11.1 /  3.8 /  4.7    128 x 64 x 1943 TN   41.5 /  7.2 / 10.4
 //   1151 x 102 x 2320 NN 70.8 / 15.6 / 11.5    224 x 704 x 2256 NN  34.6 / 14.8 / 14.5
 //   512^3 NT              6.5 /  8.7 /  5.6    1000 x 500 x 300 TT  10.6 /  7.3 /  6.0
+//   512 x 640 x 1024 NT   9.6 /        11.9    512 x 640 x 1024 TN  17.1 /        10.0
 //   640 x 640 x 1280 TN  21.0 / 23.7 / 10.3    768^3 NT              8.2 / 16.6 / 12.1
 // A wave sums a quarter of K in one accumulator, the tiled kernels' k-slices
 // 1024 k and more each: where those slice, K ends at 4096, beyond which this
@@ -191,7 +193,8 @@ bool gemm_direct16_ok(const GemmArgs& g) {
     const bool whole = g.M % 64 == 0 && g.N % 64 == 0 && g.K % 64 == 0 && g.lda % 8 == 0 &&
                        g.ldb % 8 == 0 && (uintptr_t)g.A % 16 == 0 && (uintptr_t)g.B % 16 == 0;
     if (g.K > 4096 && splitk_applies(tiles_of(g, 64), g.K)) return false;
-    return tiles_of(g, 32) <= (whole ? 320 : 768);
+    const bool tn = g.opA == CDX_OP_T && g.opB == CDX_OP_N;
+    return tiles_of(g, 32) <= (!whole ? 768 : tn ? 320 : 256);
 }
 
 int launch_gemm_direct16(const GemmArgs& g, bool bf16, hipStream_t stream) {
