@@ -210,7 +210,17 @@ int64_t tiles_of(const GemmArgs& g, int64_t side) {
 //   1024^3 NN           28.7      39.9       48.1       25.7
 //   8192 x 256 x 784 NT 38.9      60.6       67.2       31.8
 // so: all products of up to 400 32 x 32 tiles, and beyond that those whose
-// rows or k the tiled kernel would have to check element by element.
+// rows or k the tiled kernel would have to check element by element, up to
+// where its larger tiles win even so (k past the last 16 alone costs it least;
+// a short k and a transposed A cost this kernel most; M or N up to 64 has its
+// own wide tiles there).  Tiled / this, us:
+//   1600 x 1600 x 300 NT 32.1 / 28.4 (1600 tiles)   1999 x 1501 x 701 NT   89.7 / 56.3 (2961)
+//   1601^2 x 61 NN       15.9 / 13.5 (2601)         1999 x 1501 x 701 TN   66.9 / 66.9
+//   1601^2 x 127 NT      19.6 / 23.2                8192 x 300 x 100 TN    13.2 / 16.4 (2560)
+//   4160 x 384 x 680 TN  33.8 / 37.8 (1560)         61 x 100001 x 300 NN   61.9 / 91.0 (6252)
+//   548 x 4441 x 120 NN  16.7 / 15.5 (2502)         14912 x 196 x 2302 NN  235 / 177 (3262)
+//   NCHW map, with the im2col before it: 96 x 13456 x 585 52.8 / 46.6 (1263),
+//   200 x 7688 x 549 49.7 / 52.8 (1687), 256 x 26912 x 459 104.5 / 133.3 (6728)
 // 64-row NN products and the convolutions' output map keep one k order, that
 // of the tiled kernels, so that the same column of a wider product (another
 // round of images) is the same bits.
@@ -223,8 +233,15 @@ bool gemm_direct_ok(const GemmArgs& g) {
     if (g.batch == 1 && splitk_applies(ceil_div(g.M, 64) * ceil_div(nb, 64), g.K)) return false;
     const int64_t t32 = tiles_of(g, 32);
     if (t32 <= 400) return true;
+    if (t32 > (g.K >= 128 ? 4096 : 3000)) return false;
     const KParams kp = f32::kparams_of(g, g.K);
-    return t32 <= 8192 && !(kp.vec_a && kp.vec_b && g.K % 16 == 0);
+    const bool tn = g.opA == CDX_OP_T && g.opB == CDX_OP_N, nt = g.opA == CDX_OP_N && g.opB == CDX_OP_T;
+    if (kp.vec_a && kp.vec_b) return g.K % 16 != 0 && (t32 <= 1024 || (t32 <= 1700 && !tn && g.n_split == 0));
+    if (t32 <= 1700) return true;
+    if (g.n_split > 0 || tn || g.M <= 64 || nb <= 64) return false;
+    const bool neither = !kp.vec_a && !kp.vec_b;
+    if (g.K < 128) return !nt && (neither || g.K >= 32);
+    return neither || g.opA == CDX_OP_N;
 }
 
 // In the TF32 modes (exact fp32 products are inside their error bar): while

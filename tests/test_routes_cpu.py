@@ -23,3 +23,27 @@ from tests.routes import gemm_kernel
 ])
 def test_gemm16(kind, M, N, K, tA, tB, want):
     assert gemm_kernel(kind, M, N, K, tA, tB) == want
+
+
+@pytest.mark.parametrize("M,N,K,tA,tB,want", [
+    (640, 640, 512, False, False, "direct"),      # up to 400 tiles of 32 x 32
+    (640, 672, 512, False, False, "tiled"),
+    (1024, 1024, 100, True, False, "direct"),     # only k ragged: 1024 tiles, 1700 unless TN
+    (1280, 1280, 300, False, True, "direct"),
+    (1280, 1280, 300, True, False, "tiled"),
+    (1600, 1600, 300, False, True, "tiled"),
+    (1301, 1301, 90, True, False, "direct"),      # rows ragged: 1700
+    (1601, 1601, 61, False, False, "direct"),     # beyond, by k and orientation
+    (1601, 1601, 127, False, True, "tiled"),
+    (1601, 1601, 701, False, True, "direct"),
+    (1601, 1601, 701, True, False, "tiled"),
+    (61, 100001, 301, False, False, "tiled"),     # one side within 64: wide tiles there
+    (100001, 61, 301, False, True, "tiled"),
+    (548, 4441, 120, False, False, "direct"),
+    (548, 4441, 20, False, False, "tiled"),
+    (14912, 196, 2302, False, False, "direct"),
+    (90, 50001, 301, False, True, "tiled"),       # more than 4096 tiles
+    (90, 40001, 101, False, False, "tiled"),      # more than 3000
+])
+def test_gemm_f32_direct(M, N, K, tA, tB, want):
+    assert gemm_kernel(0, M, N, K, tA, tB) == want
