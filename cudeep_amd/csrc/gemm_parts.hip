@@ -473,9 +473,37 @@ Slices slices_of(const GemmArgs& g) {
 
 }  // namespace
 
+namespace {
+
+// Unsliced products: whether this kernel's rounds of one workgroup per CU beat
+// the tiled fp32 kernel's rounds of 64 x 64 tiles.  Both costs are in us, from
+// fits to whole tiles with 16-byte rows; A transposed costs this kernel more,
+// ragged sizes and rows cost the tiled one more.  Within an eighth this kernel
+// is taken, for its smaller error.  Tiled / this, us:
+//   4096 x 4096 x 48 NN   37 / 57    2048 x 2304 x 64 NN     11 / 18
+//   2048 x 2048 x 64 NN   10 / 11    2048 x 2304 x 512 NN    46 / 52
+//   2048 x 2048 x 128 NN  14 / 14    2048 x 2304 x 2048 NN  167 / 179
+//   3072 x 3072 x 64 NN   18 / 26    2048 x 2304 x 2048 TN  166 / 210
+//   3072 x 3072 x 512 NN  80 / 79    2999 x 1501 x 2048 TN  291 / 200
+//   8192 x 784 x 256 NN   35 / 34    2501 x 2503 x 128 NN    33 / 27
+// (the slow ones: a pipeline's filling over a k-tile or four, and a second
+// round of 32 workgroups)
+bool beats_tiled(const GemmArgs& g, int64_t tiles) {
+    const KParams kp = f32::kparams_of(g, g.K);
+    const int64_t nb = g.ones_col >= 0 ? g.ones_col : g.N;
+    const double rounds = (double)ceil_div(tiles * g.batch, 256);
+    const double rounds64 = (double)ceil_div(ceil_div(g.M, 64) * ceil_div(nb, 64) * g.batch, 256);
+    const bool whole = g.M % 64 == 0 && nb % 64 == 0;
+    const double slow = !kp.vec_a && !kp.vec_b ? 1.7 : !kp.vec_a || !kp.vec_b ? 1.35 : g.K % 16 != 0 ? 1.2 : whole ? 1.0 : 1.1;
+    const double parts = 3.0 + rounds * (5.0 + (g.opA == CDX_OP_T ? 1.5 : 1.25) * (double)ceil_div(g.K, PBK));
+    return parts <= 1.12 * (6.0 + 0.5 * slow * rounds64 * (double)g.K / PBK);
+}
+
+}  // namespace
+
 // Which products: those with a 128 x 128 tile for nearly every CU (2048^3 92
-// against 131 us on the fp32 matrix path, 8192 x 784 x 256 33 against 36, 5079
-// x 896 x 920 NT 88 against 93), or with enough k-slices of such tiles (256 x
+// against 131 us on the fp32 matrix path, 5079 x 896 x 920 NT 88 against 93)
+// unless beats_tiled() says otherwise, or with enough k-slices of such tiles (256 x
 // 785 x 8192 TN 38 against 49; 2539 x 704 x 2624 NT 76 against 124; 512 x 1024
 // x 8192 TN 67 against 181; 64 workgroups, 256 x 257 x 4096 TN, 24 against 22).
 // With fewer tiles and a short K the smaller fp32 tiles win: 8192 x 256 x 784
@@ -489,7 +517,7 @@ bool gemm_parts_ok(const GemmArgs& g) {
         return false;
     const int64_t tiles = own_tiles(g);
     if (tiles > INT32_MAX / 2 || tiles * (PTile::BM * PTile::BN) > g.M * nb / 5 * 7) return false;
-    if (tiles >= 240) return true;
+    if (tiles >= 240) return beats_tiled(g, tiles);
     const int n = slices_of(g).n;
     return n > 1 && tiles * n >= 160;
 }

@@ -26,6 +26,24 @@ def test_gemm16(kind, M, N, K, tA, tB, want):
 
 
 @pytest.mark.parametrize("M,N,K,tA,tB,want", [
+    (2048, 2048, 48, False, False, "tiled"),      # short k: the pipeline only fills
+    (2048, 2048, 128, False, False, "parts"),
+    (4096, 4096, 48, False, True, "tiled"),
+    (4096, 4096, 512, False, True, "parts"),
+    (25088, 392, 32, False, False, "tiled"),
+    (2048, 2304, 64, False, False, "tiled"),      # 288 tiles: a second round of 32
+    (2048, 2304, 2048, False, False, "parts"),
+    (2048, 2304, 2048, True, False, "tiled"),
+    (2999, 1501, 2048, True, False, "parts"),     # rows the tiled kernel reads one by one
+    (8192, 784, 256, False, False, "parts"),
+    (4096, 4096, 4096, True, True, "parts"),
+    (256, 785, 8192, True, False, "parts"),       # k-slices
+])
+def test_gemm_f32_parts(M, N, K, tA, tB, want):
+    assert gemm_kernel(0, M, N, K, tA, tB) == want
+
+
+@pytest.mark.parametrize("M,N,K,tA,tB,want", [
     (640, 640, 512, False, False, "direct"),      # up to 400 tiles of 32 x 32
     (640, 672, 512, False, False, "tiled"),
     (1024, 1024, 100, True, False, "direct"),     # only k ragged: 1024 tiles, 1700 unless TN
