@@ -19,19 +19,26 @@
 // 2048^3 1.3e-7 (8.1e-7), 8192 x 784 x 256 6.4e-8 (2.9e-7), 256 x 785 x 8192
 // in k-slices 1.6e-7 (3.2e-7).
 //
-// Range.  The parts are exact while l stays above bf16's smallest magnitude,
-// i.e. for |x| >= 2^-110 (or 0), and finite for |x| below bf16's rounding
-// limit.  An output can lose accuracy only if every |a| of its row (or |b| of
-// its column) is below 2^-110; with the other operand below 2^40 and K <=
-// 2^16 such an output is below 2^-54; it is zero only if subnormals vanished.
-// So a workgroup recomputes its tile with the fp32 matrix instruction
-// (f32::gemm_tile, the same arithmetic as gemm_f32.hip) when it staged an
-// |x| >= 2^40 (infinities among them), or some accumulator is NaN, or nonzero
-// and below 2^-54, or zero where a subnormal was staged.  On data without such
-// values this costs four VALU operations per two staged elements and four
-// compares per output (8192 x 784 x 256 33.3 us against 32.6 without the search
-// for subnormals, 4096^3 the same; a class compare per element instead 36, and
-// a second pass over the operands of tiles with a zero output 43 with zero rows).
+// Range.  The parts are exact for |x| >= 2^-110 (or 0), where l stays above
+// bf16's smallest normal magnitude, and finite below bf16's rounding limit.  A
+// smaller x loses at most 2^-125, and a product of parts that the matrix core
+// flushes 2^-126.  So nothing is lost to speak of while the least magnitudes of
+// both operands (0 aside) are at least 2^-110 and their product 2^-98 (2^-28
+// of each product); else an output is off by at most K 2^-125 max|x| + K 6
+// 2^-126, 2^-25 of one of K 2^-100 max|x| + 2^-80 or more, and it is 0 by mistake only
+// if subnormals were staged or the least product is below 2^-125.  A workgroup
+// recomputes its tile with the fp32 matrix instruction (f32::gemm_tile, the
+// same arithmetic as gemm_f32.hip) when some accumulator is infinite or NaN, or
+// in those last two cases; the block-wide extremes they need are formed only
+// when an output is below 2^-43 (or an |x| at least 2^40) and an operand below
+// 2^-49.  A recomputed product costs both kernels.  us, the fp32 kernel's / this
+// one's: 4096^3 with a row of 1e-18, one 2^41 per panel or a mask of -1e30
+// 980 / 705-737, 8192 x 784 x 256 35 / 33, as for N(0, 1); recomputed, with a
+// mask of -infinity or both operands scaled by 2^-40, 970 / 2250 and 35 / 90.
+// Looking costs four VALU operations per two staged elements and two compares
+// per output (8192 x 784 x 256 33.3 us against 32.6 without the search for the
+// least; a class compare per element instead 36, and a second pass over the
+// operands of tiles with a zero output 43 with zero rows).
 //
 // Structure (per workgroup, one 128 x 128 output tile, k-tiles of 32): eight
 // waves in two groups of four, one wave of each per SIMD.  Each group owns the
@@ -89,6 +96,15 @@ __device__ __forceinline__ void split3(float a, float b, uint32_t& h, uint32_t& 
     const float ra = a - lo(h), rb = b - hi(h);
     m = pk(ra, rb);
     l = pk(ra - lo(m), rb - hi(m));
+}
+
+// Magnitudes but 0 in order, from a float's bits; that of 2^e; and back.
+__device__ __forceinline__ constexpr uint32_t least_code(uint32_t bits) { return (bits << 1) - 1u; }
+__device__ __forceinline__ constexpr uint32_t least_code_exp2(int e) {
+    return least_code((uint32_t)(e + 127) << 23);
+}
+__device__ __forceinline__ float least_value(uint32_t code) {   // (none seen: the largest)
+    return code == 0xffffffffu ? 3.4028235e38f : __builtin_bit_cast(float, (code >> 1) + 1u);
 }
 
 // One operand's k-tile: BMN rows (m or n) x 32 k as 4 x 4 blocks (the walk of
@@ -177,8 +193,8 @@ struct PartLoader {
         }
     }
     // Splits into the three planes at s ([mn][PSTRIDE], `plane` apart);
-    // amax: the largest magnitude seen; least: the smallest but 0, as its bits
-    // without the sign, doubled, less one.
+    // amax: the largest magnitude seen; least: the smallest but 0, as
+    // least_code() (0's wraps round to the largest).
     __device__ __forceinline__ void store(unsigned short* s, int plane, float& amax,
                                           uint32_t& least, int tid) const {
 #pragma unroll
@@ -194,7 +210,7 @@ struct PartLoader {
                 asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(amax) : "v"(x.z), "v"(x.w));
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    const uint32_t u = (__builtin_bit_cast(uint32_t, x[i]) << 1) - 1u;
+                    const uint32_t u = least_code(__builtin_bit_cast(uint32_t, x[i]));
                     least = u < least ? u : least;
                 }
                 uint2 h, m, l;
@@ -209,9 +225,6 @@ struct PartLoader {
     }
 };
 
-// (the outputs and operands a tile is recomputed for: see Range above)
-constexpr float kPartsHuge = 0x1p40f, kPartsTiny = 0x1p-54f;
-
 template <int OPA, int OPB>
 __global__ __launch_bounds__(PTile::NT)
 void gemm_parts_kernel(KParams p) {
@@ -222,7 +235,8 @@ void gemm_parts_kernel(KParams p) {
     constexpr int STAGE = 3 * (A_PLANE + B_PLANE);   // bf16
     using Fallback = CF::Fallback;
     __shared__ __attribute__((aligned(16))) unsigned short lds[2 * STAGE];
-    __shared__ int redo, subnormals, zeros;
+    __shared__ int redo, small_out, small_in;
+    __shared__ uint32_t ext[3];   // least of A, of B; largest of both (bits)
     static_assert(2 * STAGE * 2 >= 8 * 8 * 64 * 16, "the hand-over needs 64 KiB");
     static_assert(2 * STAGE * 2 >= f32::Geo<Fallback, OPA, OPB>::LDS_FLOATS * 4, "fallback tile");
 
@@ -276,13 +290,13 @@ void gemm_parts_kernel(KParams p) {
         else if (t < nk) lb.load_tail(pb + t * step_b, p.ldb, krem, tid);
     };
     float amax = 0.0f;
-    uint32_t least = 0xffffffffu;
+    uint32_t least_a = 0xffffffffu, least_b = 0xffffffffu;
     auto store = [&](int64_t t) {
         const int kr = t + 1 < nk ? PBK : krem;
         if (edge_a || kr < PBK) la.fix(arem, kr, -1, tid);
-        la.store(sA, A_PLANE, amax, least, tid);
+        la.store(sA, A_PLANE, amax, least_a, tid);
         if (edge_b || kr < PBK) lb.fix(brem, kr, one, tid);
-        lb.store(sB, B_PLANE, amax, least, tid);
+        lb.store(sB, B_PLANE, amax, least_b, tid);
     };
 
     floatx4 acc[FM][FN];
@@ -345,7 +359,11 @@ void gemm_parts_kernel(KParams p) {
 
     // group g takes the k-tiles g, g + 2, ...; both run the barriers of the
     // longer list, group 1 one slot behind
-    if (threadIdx.x == 0) redo = subnormals = zeros = 0;
+    if (threadIdx.x == 0) {
+        redo = small_out = small_in = 0;
+        ext[0] = ext[1] = 0xffffffffu;
+        ext[2] = 0u;
+    }
     const int64_t slots = (nk + 1) / 2;
     if (grp < nk) {
         load_a(grp);
@@ -395,22 +413,46 @@ void gemm_parts_kernel(KParams p) {
                 res[i][j] = red[((w * 2 + 1) * 8 + i * FN + j) * 64 + lane] + acc[2 + i][j];
     }
 
-    bool bad = !(amax < kPartsHuge), zero = false;
+    // Recompute? (see Range above.)  Values that are lost need a small operand
+    // and show in a small output, or one beside operands that are very large.
+    auto any_output = [&](auto&& of) {
+        bool any = false;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j)
+            for (int j = 0; j < FN; ++j)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float c = __builtin_fabsf(res[i][j][e]);
-                bad |= !(c >= kPartsTiny) && c != 0.0f;   // NaN too
-                zero |= c == 0.0f;
-            }
-    if (bad) redo = 1;
-    if (zero) zeros = 1;
-    if (least < (2u << 23) - 1u) subnormals = 1;   // (that of 2^-126)
+                for (int e = 0; e < 4; ++e) any |= of(__builtin_fabsf(res[i][j][e]));
+        return any;
+    };
+    if (any_output([](float c) { return !(c <= 3.4028235e38f); })) redo = 1;   // NaN too
+    if (any_output([](float c) { return c < 0x1p-43f; }) || !(amax < 0x1p40f)) small_out = 1;
+    if (least_a < least_code_exp2(-49) || least_b < least_code_exp2(-49)) small_in = 1;
     __syncthreads();
-    if (redo || (zeros && subnormals)) {   // (uniform) the fp32 matrix path, a smaller tile at a time
+    if (!redo && small_out && small_in) {   // (uniform)
+        uint32_t top = __builtin_bit_cast(uint32_t, amax);
+        for (int d = 32; d > 0; d >>= 1) {
+            const uint32_t a = __shfl_xor(least_a, d), b = __shfl_xor(least_b, d), t = __shfl_xor(top, d);
+            least_a = a < least_a ? a : least_a;
+            least_b = b < least_b ? b : least_b;
+            top = t > top ? t : top;
+        }
+        if (lane == 0) {
+            atomicMin(&ext[0], least_a);
+            atomicMin(&ext[1], least_b);
+            atomicMax(&ext[2], top);
+        }
+        __syncthreads();
+        const uint32_t lo = ext[0] < ext[1] ? ext[0] : ext[1];
+        const float least_product = least_value(ext[0]) * least_value(ext[1]);
+        if (lo < least_code_exp2(-110) || least_product < 0x1p-98f) {
+            const float bound = 0x1p-80f + 0x1p-100f * (float)p.K * __builtin_bit_cast(float, ext[2]);
+            const bool zeros = lo < least_code_exp2(-126) || least_product < 0x1p-125f;
+            if (any_output([&](float c) { return c == 0.0f ? zeros : c < bound; })) redo = 1;
+        }
+        __syncthreads();
+    }
+    if (redo) {   // (uniform) the fp32 matrix path, a smaller tile at a time
         constexpr int TN = BN / Fallback::BN;
 #pragma unroll 1
         for (int s = 0; s < BM / Fallback::BM * TN; ++s) {

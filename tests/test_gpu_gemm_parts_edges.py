@@ -94,3 +94,75 @@ def test_batch():
         ref = want[:, ::97].cpu()
         e_ref = float((one.double() - ref).norm() / ref.norm())
         assert float((y[b].double() - want).norm() / want.norm()) <= 2 * e_ref
+
+
+# (the value, its row and column in A: 2^41 and a mask's -1e30 among N(0, 1), or a whole row)
+@pytest.mark.parametrize("what", ["2^41", "-1e30", "1e-18 row", "1e30 in B", "zero and tiny rows"])
+def test_outliers_leave_the_other_rows_alone(what):
+    """One large value, or a row of small ones, does not send the tile's other outputs to the
+    fp32 matrix path: they are the same bits as without it, and the row itself meets its bar."""
+    import torch
+    M, N, K = 2048, 2048, 160
+    assert gemm_kernel(0, M, N, K) == "parts"
+    rng = np.random.default_rng(21)
+    A, B = normal(rng, (M, K)), normal(rng, (K, N))
+    say("gemm parts outliers", what)
+    base = ops().gemm(dev(A), dev(B))
+    rows, cols = [5], []
+    if what == "2^41":
+        # (1.37: with a power of two the one large product is exact in the reference, whose error
+        # is then not a rounding, 2^-24, but only what the rest of the sum is worth, 2^-37)
+        A[5, 7] = 1.37 * 2.0 ** 41
+    elif what == "-1e30":
+        A[5, ::3] = -1e30
+    elif what == "1e30 in B":
+        B[7, 9] = 1e30
+        rows, cols = [], [9]
+    elif what == "1e-18 row":
+        A[5] *= np.float32(1e-18)
+    else:
+        A[5] *= np.float32(1e-18)
+        A[64:96] = 0.0
+        rows = [5] + list(range(64, 96))
+    C = ops().gemm(dev(A), dev(B))
+    same = torch.ones((M, N), dtype=torch.bool, device="cuda")
+    same[rows, :] = False
+    same[:, cols] = False
+    assert torch.equal(C[same], base[same])
+    _check(host(C), A, B, False, False, [5])
+    assert what != "zero and tiny rows" or not host(C)[64:96].any()
+
+
+@pytest.mark.parametrize("sa,sb", [(-70, -44), (-109, -9), (-100, 2), (-60, -40), (100, -80),
+                                   (-112, 60), (30, -111)])
+def test_scales(sa, sb):
+    """Operands scaled by powers of two on either side of the lines at which parts or their
+    products would vanish, with values of other sizes beside them: every row to the bar."""
+    M, N, K = 2048, 2048, 160
+    rng = np.random.default_rng(22)
+    A = (normal(rng, (M, K)).astype(np.float64) * 2.0 ** sa).astype(np.float32)
+    B = (normal(rng, (K, N)).astype(np.float64) * 2.0 ** sb).astype(np.float32)
+    A[9] *= np.float32(2.0 ** -12)
+    A[140, 3] *= np.float32(2.0 ** 20)
+    say("gemm parts scales", sa, sb)
+    C = host(ops().gemm(dev(A), dev(B)))
+    for rows in ([9], [140], list(range(16, 40))):
+        _check(C, A, B, False, False, rows)
+
+
+def test_infinite_and_overflowing_outputs():
+    """Infinities, NaN, sums that overflow and values that bf16 would round to infinity: IEEE."""
+    M, N, K = 2048, 2048, 160
+    rng = np.random.default_rng(23)
+    A, B = normal(rng, (M, K)), normal(rng, (K, N))
+    A[3, 5], A[300, 9], A[600, 11] = np.inf, np.nan, 3.4028234e38
+    A[900, :2], B[:2, 40] = 3e38, 1.0
+    B[11] = 0.5
+    say("gemm parts infinities")
+    C = host(ops().gemm(dev(A), dev(B)))
+    with np.errstate(invalid="ignore", over="ignore"):
+        C64 = A.astype(np.float64) @ B.astype(np.float64)
+    assert np.array_equal(np.isnan(C), np.isnan(C64))
+    assert np.array_equal(np.sign(C[3]), np.sign(C64[3])) and np.isinf(C[3]).all()
+    assert np.isposinf(C[900, 40])
+    _check(C, A, B, False, False, [600])
