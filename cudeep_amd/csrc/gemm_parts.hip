@@ -8,16 +8,26 @@
 // where both differences are exact and l has at most 8 significant bits, so
 // x = h + m + l exactly, and
 //     a b = ah bh + (ah bm + am bh) + (am bm + ah bl + al bh)  +  r
-// with |r| <= 2^-25 |ab| (am bl + al bm + al bl: |m| <= 2^-9 |x|, |l| <=
-// 2^-18 |x|), below half an fp32 rounding of the product.  The six products
-// of a 32-k step are summed from zero, small ones first, and added to the
-// accumulator by an fp32 add: added by the matrix instruction itself, whose
-// sums round towards one side, the errors of a column of outputs all lean the
-// same way (relative Frobenius error 1.00e-6 at 4096^3, most of it bias; the
-// column sums off by 1.3e-5).  Relative Frobenius error against fp64, N(0, 1)
-// operands (in brackets the fp32-MFMA kernels'): 4096^3 1.7e-7 (1.15e-6),
-// 2048^3 1.3e-7 (8.1e-7), 8192 x 784 x 256 6.4e-8 (2.9e-7), 256 x 785 x 8192
-// in k-slices 1.6e-7 (3.2e-7).
+// with |r| <= 2^-24 |ab|, 2^-27 in the mean square (am bl + al bm + al bl: |m| <=
+// 2^-8 |x|, |l| <= 2^-17 |x|).  The six products of a 32-k step are summed from
+// zero, small ones first, and added to the accumulator by an fp32 add: added by
+// the matrix instruction itself, whose sums round towards one side, the errors
+// of a column of outputs all lean the same way (relative Frobenius error 1.00e-6
+// at 4096^3, most of it bias; the column sums off by 1.3e-5).  Relative Frobenius
+// error against fp64, N(0, 1) operands (in brackets the fp32-MFMA kernels'):
+// 4096^3 1.7e-7 (1.15e-6), 2048^3 1.3e-7 (8.1e-7), 8192 x 784 x 256 6.4e-8
+// (2.9e-7), 256 x 785 x 8192 in k-slices 1.6e-7 (3.2e-7).
+//
+// Sparse rows are where it is the less exact one.  The fp32 matrix instruction
+// forms a product whole and rounds to nearest; here r is left out and the
+// largest term is added with a one-sided rounding, so an output that is one
+// product is off by up to 2^-23 + 2^-24 instead of 2^-24.  2048^3, N(0, 1)
+// nonzeros, in brackets the fp32-MFMA kernels': a diagonal A 3.5e-8 (2.5e-8; at
+// most 2^-22.6 of an output against 2^-24), 3 per row 5.1e-8 (3.6e-8), 8 6.5e-8
+// (5.4e-8), 16 7.8e-8 (7.4e-8), 30 9.3e-8 (9.9e-8); identities, permutations and
+// powers of two are exact.  With h h in an accumulator of its own, added to the
+// others' sum by fp32 adds, a diagonal A is at 2.6e-8 and three per row at
+// 4.3e-8, for 5 % more time (4096^3 731 -> 775 us, 2048^3 94 -> 100).
 //
 // Range.  The parts are exact for |x| >= 2^-110 (or 0), where l stays above
 // bf16's smallest normal magnitude, and finite below bf16's rounding limit.  A

@@ -166,3 +166,28 @@ def test_infinite_and_overflowing_outputs():
     assert np.array_equal(np.sign(C[3]), np.sign(C64[3])) and np.isinf(C[3]).all()
     assert np.isposinf(C[900, 40])
     _check(C, A, B, False, False, [600])
+
+
+@pytest.mark.parametrize("tA,tB", [(False, False), (True, True)])
+def test_one_product_per_output(tA, tB):
+    """A diagonal, a permutation and powers of two.  An output that is one product ab misses the
+    terms am bl + al bm + al bl, at most 2^-24 |ab|, and takes one rounding to one side, 2^-23, on
+    the sum's way to 24 bits (the smaller terms' own roundings are 2^-8 of that); with one factor a
+    power of two its m and l are 0 and nothing is lost."""
+    M = N = K = 2048
+    assert gemm_kernel(0, M, N, K, tA, tB) == "parts"
+    rng = np.random.default_rng(31)
+    B = normal(rng, (K, N))
+    perm = rng.permutation(K)
+
+    def product(A):
+        return host(ops().gemm(dev(A.T if tA else A), dev(B.T if tB else B), transA=tA, transB=tB))
+    say("gemm parts one product per output", tA, tB)
+    d = normal(rng, (K,))
+    want = d.astype(np.float64)[:, None] * B
+    off = np.abs(product(np.diag(d)) - want)
+    assert (off <= (2.0 ** -23 + 2.0 ** -24 + 2.0 ** -31) * np.abs(want)).all()
+    A = np.zeros((M, K), np.float32)
+    A[np.arange(M), perm] = np.exp2(rng.integers(-20, 20, M)).astype(np.float32) * \
+        rng.choice([-1, 1], M).astype(np.float32)
+    assert np.array_equal(product(A), A[np.arange(M), perm][:, None] * B[perm])
