@@ -172,9 +172,13 @@ int launch_cfg(const GemmArgs& g, hipStream_t stream) {
     const KParams kp = f32::kparams_of(g, g.K);
     const int64_t tiles = ceil_div(g.M, 16 * FM * WM) * ceil_div(g.N, 16 * FN * WN);
     const dim3 grid((unsigned)tiles, 1, (unsigned)g.batch), block(256);
-    if (g.n_split > 0)
-        hipLaunchKernelGGL((gemm_direct_kernel<FM, FN, WM, WN, WK, CDX_OP_N, CDX_OP_N, true>), grid, block, 0, stream, kp);
-    else if (g.opA == CDX_OP_N && g.opB == CDX_OP_N)
+    if constexpr (WK == 1) {   // (the NCHW map keeps one k order: launch_gemm_direct)
+        if (g.n_split > 0) {
+            hipLaunchKernelGGL((gemm_direct_kernel<FM, FN, WM, WN, WK, CDX_OP_N, CDX_OP_N, true>), grid, block, 0, stream, kp);
+            return hip_error(hipGetLastError(), "gemm_direct_kernel launch");
+        }
+    }
+    if (g.opA == CDX_OP_N && g.opB == CDX_OP_N)
         hipLaunchKernelGGL((gemm_direct_kernel<FM, FN, WM, WN, WK, CDX_OP_N, CDX_OP_N, false>), grid, block, 0, stream, kp);
     else if (g.opA == CDX_OP_N)
         hipLaunchKernelGGL((gemm_direct_kernel<FM, FN, WM, WN, WK, CDX_OP_N, CDX_OP_T, false>), grid, block, 0, stream, kp);
