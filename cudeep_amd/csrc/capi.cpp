@@ -183,25 +183,49 @@ bool forward_few_columns(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int6
     return col_bytes(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW) <= ((size_t)4 << 20);
 }
 
+// Whether the implicit forward GEMM of a layer runs on the kernel whose waves
+// gather their own operands (conv_direct.hip), else on the row-window kernel
+// or, where its window does not fit LDS, the gathering one (conv_implicit.hip).
+bool implicit_is_direct(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH,
+                        int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
+    return cdx::conv_direct_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW) &&
+           cdx::conv_direct_pays(batch * conv_out(IH, KH, SH, PH) * conv_out(IW, KW, SW, PW), OC,
+                                 IC * KH * KW,
+                                 cdx::conv_rowwin_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW));
+}
+
 // The forward dispatch below the Winograd route.  The reference sends a layer
 // whose column buffer would exceed 4 MiB to its implicit kernel (no buffer;
-// conv_kernel.cu:242-275); here every layer takes the implicit GEMM unless it
-// is a 3x3 stride-1 layer with >= 16 output pixels per image (the Winograd
-// shape, which keeps the im2col route here when it is not sent to Winograd):
-// below 4 MiB of columns one launch beats im2col + GEMM as well (6 x 56 -> 46,
-// 31^2, 3x3 stride 2: 16 -> 11 us; 3 x 168 -> 99, 56^2, 1x1 stride 2: 13 ->
-// 9), and its products are fp32 in every precision mode.  The reference's
-// naive-kernel shapes (K_col < 9 or fewer than 4 output pixels per image,
-// checked before the implicit route at conv_kernel.cu:250) take the im2col
-// route, which computes the same sums.
-bool forward_takes_implicit(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int64_t KH,
-                            int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
+// conv_kernel.cu:242-275) unless it is a 3x3 stride-1 layer with >= 16 output
+// pixels per image (the Winograd shape, which keeps the im2col route here when
+// it is not sent to Winograd).  The reference's naive-kernel shapes (K_col < 9 or
+// fewer than 4 output pixels per image, checked before the implicit route at
+// conv_kernel.cu:250) take the im2col route, which computes the same sums.  All
+// other layers have fp32 products in every precision mode, on whichever route.
+bool forward_is_fp32(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int64_t KH, int64_t KW,
+                     int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
     const int64_t OH = conv_out(IH, KH, SH, PH), OW = conv_out(IW, KW, SW, PW);
     const bool s3 = KH == 3 && KW == 3 && SH == 1 && SW == 1;
     if (s3 && (OH * OW >= 16 || forward_few_columns(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW)))
         return false;
-    if (IC * KH * KW < 9 || OH * OW < 4) return false;
-    return cdx::conv_fwd_implicit_ok(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW);
+    return IC * KH * KW >= 9 && OH * OW >= 4 &&
+           cdx::conv_fwd_implicit_ok(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW);
+}
+
+// Of those, the ones on the implicit GEMM.  Below 4 MiB of columns one launch of
+// the direct kernel beats im2col + GEMM as well (6 x 56 -> 46, 31^2, 3x3 stride
+// 2: 16 -> 11 us; 3 x 168 -> 99, 56^2, 1x1 stride 2: 13 -> 9), but not beyond
+// 3200 k, where the column route's product runs in slices (im2col + GEMM /
+// direct: 1 x 128 -> 64, 28^2, 5x5 stride 2, 3200 k 29 / 29; 1 x 200 -> 64, 13^2,
+// 5x5, 5000 k 31 / 44; 2 x 200 -> 48, 14^2, 7x7 stride 2, 9800 k 36 / 84), and
+// not on the kernels that tile larger layers (4 x 256 -> 512, 56^2, 1x1 stride 2
+// 23 / 71; 1 x 128 -> 168, 13^2, 11x11 stride 4 48 / 787).
+bool forward_takes_implicit(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
+                            int64_t KH, int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
+    return forward_is_fp32(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW) &&
+           (!forward_few_columns(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW) ||
+            (IC * KH * KW <= 3200 &&
+             implicit_is_direct(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)));
 }
 
 // The workspace a forward call asks for: one round of columns, except that of
@@ -211,7 +235,7 @@ bool forward_takes_implicit(int64_t batch, int64_t IC, int64_t IH, int64_t IW, i
 size_t forward_workspace(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int64_t KH, int64_t KW,
                          int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
     if (!forward_few_columns(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW) &&
-        forward_takes_implicit(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW))
+        forward_takes_implicit(batch, IC, 1, IH, IW, KH, KW, SH, SW, PH, PW))   // (any OC)
         return 0;
     return col_round_bytes(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW);
 }
@@ -447,12 +471,8 @@ int cdx_conv2d_forward_implicit_f32(const float* input, const float* weight, con
     if (!cdx::conv_fwd_implicit_ok(batch, in_channels, in_h, in_w, kernel_h, kernel_w, stride_h,
                                    stride_w, pad_h, pad_w))
         return set_error(CDX_ERR_UNSUPPORTED, std::string(fn) + ": geometry beyond 32-bit indices");
-    if (cdx::conv_direct_ok(batch, in_channels, out_channels, in_h, in_w, kernel_h, kernel_w,
-                            stride_h, stride_w, pad_h, pad_w) &&
-        cdx::conv_direct_pays(batch * OH * OW, out_channels, in_channels * kernel_h * kernel_w,
-                              cdx::conv_rowwin_ok(batch, in_channels, out_channels, in_h, in_w,
-                                                  kernel_h, kernel_w, stride_h, stride_w, pad_h,
-                                                  pad_w)))
+    if (implicit_is_direct(batch, in_channels, out_channels, in_h, in_w, kernel_h, kernel_w, stride_h,
+                           stride_w, pad_h, pad_w))
         return cdx::launch_conv_direct_f32(input, weight, bias, output, batch, in_channels,
                                            out_channels, in_h, in_w, kernel_h, kernel_w, stride_h,
                                            stride_w, pad_h, pad_w, stream);
@@ -539,8 +559,8 @@ int cdx_conv2d_forward_f32(const float* input, const float* weight, const float*
         return set_error(CDX_ERR_INVALID_ARG, std::string(fn) + ": bad precision");
     const bool product = conv_is_product(batch, in_channels, out_channels, kernel_h, kernel_w,
                                          stride_h, stride_w, pad_h, pad_w);
-    if (product || forward_takes_implicit(batch, in_channels, in_h, in_w, kernel_h, kernel_w,
-                                          stride_h, stride_w, pad_h, pad_w)) {
+    if (product || forward_takes_implicit(batch, in_channels, out_channels, in_h, in_w, kernel_h,
+                                          kernel_w, stride_h, stride_w, pad_h, pad_w)) {
         const int64_t S = conv_out(in_h, kernel_h, stride_h, pad_h) *
                           conv_out(in_w, kernel_w, stride_w, pad_w);
         if (batch == 0 || out_channels == 0 || S == 0) return CDX_OK;
@@ -557,6 +577,9 @@ int cdx_conv2d_forward_f32(const float* input, const float* weight, const float*
                                                out_channels, in_h, in_w, kernel_h, kernel_w,
                                                stride_h, stride_w, pad_h, pad_w, stream);
     }
+    if (forward_is_fp32(batch, in_channels, in_h, in_w, kernel_h, kernel_w, stride_h, stride_w,
+                        pad_h, pad_w))
+        precision = CDX_PREC_FP32;
     return conv_forward_im2col(input, weight, bias, output, batch, in_channels, out_channels,
                                in_h, in_w, kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w,
                                precision, workspace, workspace_bytes, stream, false);
@@ -713,6 +736,14 @@ bool bwd_data_rowwin(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t 
     return cdx::conv_rowwin_ok(batch, OC, IC, OH, OW, KH, KW, 1, 1, KH - 1 - PH, KW - 1 - PW);
 }
 
+// Where such a layer runs on the direct kernel (conv_direct.hip) instead.
+bool bwd_data_is_direct(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH,
+                        int64_t KW, int64_t PH, int64_t PW) {
+    return cdx::conv_direct_pays(batch * IH * IW, IC, OC * KH * KW, true) &&
+           cdx::conv_direct_ok(batch, OC, IC, conv_out(IH, KH, 1, PH), conv_out(IW, KW, 1, PW), KH,
+                               KW, 1, 1, KH - 1 - PH, KW - 1 - PW);
+}
+
 // Workspace of the implicit backward-weight kernel (0 when it does not apply).
 size_t wgrad_implicit_floats(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
                              int64_t KH, int64_t KW, int64_t SH, int64_t SW, int64_t PH,
@@ -846,10 +877,8 @@ int cdx_conv2d_backward_data_f32(const float* grad_output, const float* weight, 
         float* wf = static_cast<float*>(ws.ptr);
         st = cdx::launch_flip_filter_f32(weight, wf, out_channels, in_channels,
                                          kernel_h * kernel_w, stream);
-        if (!st && cdx::conv_direct_pays(batch * in_h * in_w, in_channels,
-                                         out_channels * kernel_h * kernel_w, true) &&
-            cdx::conv_direct_ok(batch, out_channels, in_channels, z.OH, z.OW, kernel_h, kernel_w, 1,
-                                1, kernel_h - 1 - pad_h, kernel_w - 1 - pad_w))
+        if (!st && bwd_data_is_direct(batch, in_channels, out_channels, in_h, in_w, kernel_h,
+                                      kernel_w, pad_h, pad_w))
             st = cdx::launch_conv_direct_f32(grad_output, wf, nullptr, grad_input, batch,
                                              out_channels, in_channels, z.OH, z.OW, kernel_h,
                                              kernel_w, 1, 1, kernel_h - 1 - pad_h,
@@ -1334,4 +1363,21 @@ extern "C" const char* cdxi_gemm_kernel(int in, int opA, int opB, int64_t M, int
     if (in >= 16) return cdx::gemm_16_kernel_name(g);
     if (in == CDX_PREC_FP32) return cdx::gemm_f32_kernel_name(g);
     return cdx::gemm_bf16x3_kernel_name(g, in == CDX_PREC_TF32MODE4 ? 4 : 3);
+}
+
+// Internal: the kernel of a convolution.  `pass`: 0 cdx_conv2d_forward_f32, 1
+// cdx_conv2d_forward_implicit_f32, 2 cdx_conv2d_backward_data_f32.
+extern "C" const char* cdxi_conv_kernel(int pass, int64_t batch, int64_t IC, int64_t OC, int64_t IH,
+                                        int64_t IW, int64_t KH, int64_t KW, int64_t SH, int64_t SW,
+                                        int64_t PH, int64_t PW) {
+    const bool product = conv_is_product(batch, IC, OC, KH, KW, SH, SW, PH, PW);
+    if (pass == 2) {
+        if (!bwd_data_rowwin(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)) return "columns";
+        if (product) return "product";
+        return bwd_data_is_direct(batch, IC, OC, IH, IW, KH, KW, PH, PW) ? "direct" : "rowwin";
+    }
+    if (pass == 0 && product) return "product";
+    if (pass == 0 && !forward_takes_implicit(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)) return "im2col";
+    if (implicit_is_direct(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)) return "direct";
+    return cdx::conv_rowwin_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW) ? "rowwin" : "gather";
 }

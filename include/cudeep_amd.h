@@ -226,11 +226,12 @@ size_t cdx_conv2d_forward_workspace_size(
 /* NCHW conv forward: im2col -> one GEMM weight[OC,K_col] * col -> NCHW
  * output with the bias added in the GEMM epilogue (no transpose pass), per
  * round of images (same sums as one pass over the batch).
- * Layers other than 3x3 stride-1 ones run the implicit GEMM
- * of cdx_conv2d_forward_implicit_f32 instead (forming no columns;
- * the reference sends those beyond 4 MiB of columns to its implicit kernel,
- * conv_kernel.cu:263-275), and 1x1 stride-1 unpadded ones one product per image
- * of the tensors as they lie; both with FP32 products in every precision.
+ * Layers other than 3x3 stride-1 ones have FP32 products in every precision.
+ * Those beyond 4 MiB of columns run the implicit GEMM of
+ * cdx_conv2d_forward_implicit_f32 instead, forming no columns (the reference
+ * sends them to its implicit kernel, conv_kernel.cu:263-275), and so do smaller
+ * ones where that is the faster route; 1x1 stride-1 unpadded ones run one
+ * product per image of the tensors as they lie.
  * Replaces cudeep::kernels::launch_conv2d_forward_kernel<float>
  * (include/cudeep/kernels/conv.cuh:8-16, src/kernels/conv_kernel.cu:225-335).
  * bias may be NULL.  precision is CDX_PREC_*.  workspace may be NULL. */

@@ -12,3 +12,11 @@ def gemm_kernel(kind, M, N, K, tA=False, tB=False, lda=None, ldb=None):
     code = {"bf16": 16 + L.DTYPE_BF16, "f16": 16 + L.DTYPE_F16}.get(kind, kind)
     return f(code, int(tA), int(tB), M, N, K, lda or (M if tA else K),
              ldb or (K if tB else N)).decode()
+
+
+def conv_kernel(what, B, IC, OC, H, W, KH, KW, stride=(1, 1), pad=(0, 0)):
+    """`what`: "forward", "implicit" (the implicit forward entry point) or "data" (backward)."""
+    f = L.lib().cdxi_conv_kernel
+    f.restype, f.argtypes = ctypes.c_char_p, [ctypes.c_int] + [ctypes.c_int64] * 11
+    return f(("forward", "implicit", "data").index(what), B, IC, OC, H, W, KH, KW, *stride,
+             *pad).decode()

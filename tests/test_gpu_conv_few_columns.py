@@ -1,0 +1,38 @@
+"""Forward convolutions below 4 MiB of columns that keep the column route: a long k (the product in
+slices), layers that only the tiling implicit kernels would take, more taps than the direct kernel's
+mask.  FP32 products in every precision mode; with a caller workspace of the queried size and
+without.  Against fp64 within twice the error of the reference's own route."""
+import numpy as np
+import pytest
+
+import oracle
+from tests.gpu_util import F32_FLOOR, dev, host, normal, require_gpu, say
+from tests.routes import conv_kernel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("g", [(1, 129, 33, 14, 15, 5, 5, (2, 2), (2, 2)),
+                               (2, 70, 48, 9, 9, 7, 7, (2, 2), (3, 3)),
+                               (4, 65, 513, 56, 56, 1, 1, (2, 2), (0, 0)),
+                               (1, 12, 40, 13, 13, 11, 11, (4, 4), (5, 5))])
+@pytest.mark.parametrize("prec", [0, 1, 2])
+def test_forward(g, prec):
+    require_gpu()
+    import torch
+    import cudeep_amd.ops as ops
+    from cudeep_amd import _lib as L
+    assert conv_kernel("forward", *g) == "im2col"
+    B, IC, OC, H, W, KH, KW, stride, pad = g
+    rng = np.random.default_rng(sum(g[:7]))
+    x, w = normal(rng, (B, IC, H, W)), normal(rng, (OC, IC, KH, KW), (2.0 / (IC * KH * KW)) ** 0.5)
+    b = normal(rng, (OC,))
+    say("conv few columns", g, prec)
+    y = ops.conv2d_forward(dev(x), dev(w), dev(b), stride, pad, precision=prec)
+    y64 = oracle.conv2d_direct64(x, w, b, stride, pad)
+    ref = oracle.conv2d_ref_im2col(x, w, b, stride, pad)
+    assert oracle.rel_fro(host(y), y64) <= 2 * oracle.rel_fro(ref, y64) + F32_FLOOR
+    n = L.lib().cdx_conv2d_forward_workspace_size(B, IC, H, W, KH, KW, *stride, *pad)
+    ws = torch.full((n // 4,), float("nan"), device="cuda")
+    assert n > 0 and torch.equal(y, ops.conv2d_forward(dev(x), dev(w), dev(b), stride, pad,
+                                                       precision=prec, workspace=ws))

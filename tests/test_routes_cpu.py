@@ -1,7 +1,7 @@
 """The kernels that the library chooses (no GPU needed): both sides of each line."""
 import pytest
 
-from tests.routes import gemm_kernel
+from tests.routes import conv_kernel, gemm_kernel
 
 
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
@@ -65,3 +65,20 @@ def test_gemm_f32_parts(M, N, K, tA, tB, want):
 ])
 def test_gemm_f32_direct(M, N, K, tA, tB, want):
     assert gemm_kernel(0, M, N, K, tA, tB) == want
+
+
+# B, IC, OC, H, W, KH, KW, stride, padding
+@pytest.mark.parametrize("g,want", [
+    ((6, 56, 46, 31, 31, 3, 3, (2, 2), (1, 1)), "direct"),       # below 4 MiB of columns
+    ((3, 168, 99, 56, 56, 1, 1, (2, 2), (0, 0)), "direct"),
+    ((1, 128, 64, 28, 28, 5, 5, (2, 2), (2, 2)), "direct"),      # 3200 k
+    ((1, 129, 64, 28, 28, 5, 5, (2, 2), (2, 2)), "im2col"),
+    ((2, 200, 48, 14, 14, 7, 7, (2, 2), (3, 3)), "im2col"),
+    ((4, 256, 512, 56, 56, 1, 1, (2, 2), (0, 0)), "im2col"),     # row-window tiles enough
+    ((1, 128, 168, 13, 13, 11, 11, (4, 4), (5, 5)), "im2col"),   # more taps than a mask holds
+    ((16, 3, 64, 224, 224, 7, 7, (2, 2), (3, 3)), "gather"),     # beyond 4 MiB
+    ((2, 16, 16, 12, 12, 3, 3, (1, 1), (1, 1)), "im2col"),       # the Winograd shape
+    ((16, 256, 64, 56, 56, 1, 1, (1, 1), (0, 0)), "product"),
+])
+def test_conv_forward(g, want):
+    assert conv_kernel("forward", *g) == want
