@@ -190,7 +190,7 @@ bool implicit_is_direct(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64
                         int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
     return cdx::conv_direct_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW) &&
            cdx::conv_direct_pays(batch * conv_out(IH, KH, SH, PH) * conv_out(IW, KW, SW, PW), OC,
-                                 IC * KH * KW,
+                                 IC * KH * KW, KH * KW,
                                  cdx::conv_rowwin_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW));
 }
 
@@ -739,7 +739,7 @@ bool bwd_data_rowwin(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t 
 // Where such a layer runs on the direct kernel (conv_direct.hip) instead.
 bool bwd_data_is_direct(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH,
                         int64_t KW, int64_t PH, int64_t PW) {
-    return cdx::conv_direct_pays(batch * IH * IW, IC, OC * KH * KW, true) &&
+    return cdx::conv_direct_pays(batch * IH * IW, IC, OC * KH * KW, KH * KW, true) &&
            cdx::conv_direct_ok(batch, OC, IC, conv_out(IH, KH, 1, PH), conv_out(IW, KW, 1, PW), KH,
                                KW, 1, 1, KH - 1 - PH, KW - 1 - PW);
 }

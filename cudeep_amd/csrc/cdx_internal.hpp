@@ -285,8 +285,8 @@ int launch_conv_rowwin_f32(const float* x, const float* w, const float* bias, fl
 // the waves where the layer is small (conv_direct.hip); k summed in two levels.
 bool conv_direct_ok(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH,
                     int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW);
-// N: batch * OH * OW; rowwin: conv_rowwin_ok()
-bool conv_direct_pays(int64_t N, int64_t OC, int64_t Kc, bool rowwin);
+// N: batch * OH * OW; taps: KH * KW; rowwin: conv_rowwin_ok()
+bool conv_direct_pays(int64_t N, int64_t OC, int64_t Kc, int64_t taps, bool rowwin);
 int launch_conv_direct_f32(const float* x, const float* w, const float* bias, float* y,
                            int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
                            int64_t KH, int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW,

@@ -248,12 +248,22 @@ DirectPlan plan_of(int64_t N, int64_t OC, int64_t Kc) {
 //   32 x 256 -> 256, 14^2 (224)             112 / 117               116 / 120
 //   16 x 64 -> 64, 56^2 (448)                49 / 61
 //   16 -> 8 channels, 4 x 112^2, 5x5 (448)                           40 / 29
+// With k < 128, unsplit, 64-channel waves have too little to hide their loads
+// behind: 2 x 12 -> 512, 28^2 10.6 / 12.4, backward data 256 -> 8, 28^2 10.4 /
+// 13.1, 16 x 3 -> 64, 56^2, 5x5 s2 10.2 / 12.8 (with 32 channels 4 x 12 -> 96, 31^2
+// s2 10.9 / 8.7); except for 1x1 layers with a stride, of whose window the
+// row-window kernel uses one pixel in SH SW (4 x 96 -> 100, 56^2 s2 19 / 10).
 // Where that one's window does not fit LDS, its gathering form (64 channels x
 // 128 pixels per workgroup) keeps the layers whose k is not split here (16 x 3
-// -> 64, 224^2, 7x7 stride 2: 73 against 92).
-bool conv_direct_pays(int64_t N, int64_t OC, int64_t Kc, bool rowwin) {
-    return OC <= 16 || ceil_div(OC, 64) * ceil_div(N, 112) < 160 ||
-           (!rowwin && plan_of(N, OC, Kc).split);
+// -> 64, 224^2, 7x7 stride 2: 73 against 92) and those of 2048 tiles of this
+// kernel and more (2 x 16 -> 168, 224^2, 7x7 s2, 2352 tiles: 132 against 143; 16 x
+// 16 -> 256, 112^2, 7x7 s3, 2888: 144 against 182; 8 x 64 -> 128, 112^2, 7x7 s2,
+// 1568: 370 against 317).
+bool conv_direct_pays(int64_t N, int64_t OC, int64_t Kc, int64_t taps, bool rowwin) {
+    if (OC <= 16) return true;
+    const DirectPlan pl = plan_of(N, OC, Kc);
+    if (ceil_div(OC, 64) * ceil_div(N, 112) < 160) return Kc >= 128 || pl.fm < 4 || taps == 1;
+    return !rowwin && pl.split && ceil_div(N, 32) * ceil_div(OC, 16 * pl.fm) < 2048;
 }
 
 // 32-bit byte offsets into the input and the filter, taps within the mask.

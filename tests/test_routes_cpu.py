@@ -82,3 +82,25 @@ def test_gemm_f32_direct(M, N, K, tA, tB, want):
 ])
 def test_conv_forward(g, want):
     assert conv_kernel("forward", *g) == want
+
+
+@pytest.mark.parametrize("g,want", [
+    ((2, 12, 512, 28, 28, 3, 3, (1, 1), (1, 1)), "rowwin"),      # k < 128, 64-channel waves
+    ((16, 3, 64, 56, 56, 5, 5, (2, 2), (2, 2)), "rowwin"),
+    ((4, 12, 96, 31, 31, 3, 3, (2, 2), (1, 1)), "direct"),       # 32-channel waves
+    ((4, 96, 100, 56, 56, 1, 1, (2, 2), (0, 0)), "direct"),      # 1x1 with a stride
+    ((2, 15, 512, 28, 28, 3, 3, (1, 1), (1, 1)), "direct"),      # k = 135
+    ((2, 16, 168, 224, 224, 7, 7, (2, 2), (3, 3)), "gather"),    # 2352 tiles
+    ((8, 64, 128, 112, 112, 7, 7, (2, 2), (3, 3)), "direct"),    # 1568
+])
+def test_conv_implicit(g, want):
+    assert conv_kernel("implicit", *g) == want
+
+
+@pytest.mark.parametrize("g,want", [
+    ((2, 256, 8, 28, 28, 3, 3, (1, 1), (1, 1)), "rowwin"),       # k = 72
+    ((2, 256, 15, 28, 28, 3, 3, (1, 1), (1, 1)), "direct"),      # k = 135
+    ((98, 12, 64, 16, 16, 3, 3, (1, 1), (1, 1)), "direct"),      # 12 channels
+])
+def test_conv_backward_data(g, want):
+    assert conv_kernel("data", *g) == want
