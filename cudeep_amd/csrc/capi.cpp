@@ -247,21 +247,28 @@ size_t forward_workspace(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int6
 // products in every precision mode, as on the implicit route these layers took
 // beyond 4 MiB of columns (16 x 256 -> 64 channels at 56^2: forward 63 -> 24
 // us, backward data 51 -> 28; 14 x 53 -> 64 at 60^2: 22 -> 14, 24 -> 16).
-bool conv_is_product(int64_t batch, int64_t IC, int64_t OC, int64_t KH, int64_t KW, int64_t SH,
-                     int64_t SW, int64_t PH, int64_t PW) {
-    return KH == 1 && KW == 1 && SH == 1 && SW == 1 && PH == 0 && PW == 0 && IC > 0 && OC > 0 &&
-           batch <= 65535;
-}
-
-int conv_product(const float* w, int64_t rows, int64_t depth, const float* in, const float* bias,
-                 float* out, int64_t batch, int64_t S, bool two_level, hipStream_t stream) {
+// A product that would run in k-slices (one image, a long k) or on the kernel
+// for up to 16 rows needs scratch that a convolution's caller does not bring:
+// those stay with the implicit kernels, whose waves split k (1 x 2048 -> 64, 28^2
+// 20 us against 24 with the scratch allocated; 2048 -> 512, 7^2 17 against 25;
+// 4096 -> 64, 28^2 38 against 24).
+cdx::GemmArgs product_args(const float* w, int64_t rows, int64_t depth, const float* in,
+                           const float* bias, float* out, int64_t batch, int64_t S, bool two_level) {
     cdx::GemmArgs g{CDX_OP_N, CDX_OP_N, rows, S, depth, w, depth, in, S, out, S, 0, 0, bias,
                     bias ? CDX_BIAS_ROW : CDX_BIAS_NONE, CDX_EPI_NONE};
     g.batch = batch;
     g.stride_b = depth * S;
     g.stride_c = rows * S;
     g.blocked_sum = two_level;
-    return cdx::launch_gemm_f32(g, stream);
+    return g;
+}
+
+bool conv_is_product(int64_t batch, int64_t rows, int64_t depth, int64_t S, int64_t KH, int64_t KW,
+                     int64_t SH, int64_t SW, int64_t PH, int64_t PW, bool two_level) {
+    return KH == 1 && KW == 1 && SH == 1 && SW == 1 && PH == 0 && PW == 0 && rows > 0 && depth > 0 &&
+           batch <= 65535 && S > 0 &&
+           (batch != 1 || cdx::gemm_f32_workspace(product_args(nullptr, rows, depth, nullptr, nullptr,
+                                                               nullptr, 1, S, two_level)) == 0);
 }
 
 }  // namespace
@@ -557,12 +564,12 @@ int cdx_conv2d_forward_f32(const float* input, const float* weight, const float*
     if (st) return st;
     if (!valid_precision(precision))
         return set_error(CDX_ERR_INVALID_ARG, std::string(fn) + ": bad precision");
-    const bool product = conv_is_product(batch, in_channels, out_channels, kernel_h, kernel_w,
-                                         stride_h, stride_w, pad_h, pad_w);
+    const int64_t S = conv_out(in_h, kernel_h, stride_h, pad_h) *
+                      conv_out(in_w, kernel_w, stride_w, pad_w);
+    const bool product = conv_is_product(batch, out_channels, in_channels, S, kernel_h, kernel_w,
+                                         stride_h, stride_w, pad_h, pad_w, false);
     if (product || forward_takes_implicit(batch, in_channels, out_channels, in_h, in_w, kernel_h,
                                           kernel_w, stride_h, stride_w, pad_h, pad_w)) {
-        const int64_t S = conv_out(in_h, kernel_h, stride_h, pad_h) *
-                          conv_out(in_w, kernel_w, stride_w, pad_w);
         if (batch == 0 || out_channels == 0 || S == 0) return CDX_OK;
         if (!output || !weight || !input)
             return set_error(CDX_ERR_INVALID_ARG, std::string(fn) + ": NULL pointer");
@@ -571,8 +578,8 @@ int cdx_conv2d_forward_f32(const float* input, const float* weight, const float*
                                                 stride_h, stride_w, pad_h, pad_w))
             return set_error(CDX_ERR_WORKSPACE, std::string(fn) + ": workspace too small");
         if (product)
-            return conv_product(weight, out_channels, in_channels, input, bias, output, batch, S,
-                                false, stream);
+            return cdx::launch_gemm_f32(product_args(weight, out_channels, in_channels, input, bias,
+                                                     output, batch, S, false), stream);
         return cdx_conv2d_forward_implicit_f32(input, weight, bias, output, batch, in_channels,
                                                out_channels, in_h, in_w, kernel_h, kernel_w,
                                                stride_h, stride_w, pad_h, pad_w, stream);
@@ -857,13 +864,13 @@ int cdx_conv2d_backward_data_f32(const float* grad_output, const float* weight, 
     if (st) return st;
     if (bwd_data_rowwin(batch, in_channels, out_channels, in_h, in_w, kernel_h, kernel_w,
                         stride_h, stride_w, pad_h, pad_w) &&
-        conv_is_product(batch, in_channels, out_channels, kernel_h, kernel_w, stride_h, stride_w,
-                        pad_h, pad_w)) {
+        conv_is_product(batch, in_channels, out_channels, in_h * in_w, kernel_h, kernel_w, stride_h,
+                        stride_w, pad_h, pad_w, true)) {
         float* wt = static_cast<float*>(ws.ptr);
         st = cdx::launch_flip_filter_f32(weight, wt, out_channels, in_channels, 1, stream);
         if (!st)
-            st = conv_product(wt, in_channels, out_channels, grad_output, nullptr, grad_input, batch,
-                              in_h * in_w, true, stream);
+            st = cdx::launch_gemm_f32(product_args(wt, in_channels, out_channels, grad_output, nullptr,
+                                                   grad_input, batch, in_h * in_w, true), stream);
         return ws.release(st);
     }
     if (bwd_data_rowwin(batch, in_channels, out_channels, in_h, in_w, kernel_h, kernel_w,
@@ -1370,13 +1377,13 @@ extern "C" const char* cdxi_gemm_kernel(int in, int opA, int opB, int64_t M, int
 extern "C" const char* cdxi_conv_kernel(int pass, int64_t batch, int64_t IC, int64_t OC, int64_t IH,
                                         int64_t IW, int64_t KH, int64_t KW, int64_t SH, int64_t SW,
                                         int64_t PH, int64_t PW) {
-    const bool product = conv_is_product(batch, IC, OC, KH, KW, SH, SW, PH, PW);
+    const int64_t S = conv_out(IH, KH, SH, PH) * conv_out(IW, KW, SW, PW);
     if (pass == 2) {
         if (!bwd_data_rowwin(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)) return "columns";
-        if (product) return "product";
+        if (conv_is_product(batch, IC, OC, S, KH, KW, SH, SW, PH, PW, true)) return "product";
         return bwd_data_is_direct(batch, IC, OC, IH, IW, KH, KW, PH, PW) ? "direct" : "rowwin";
     }
-    if (pass == 0 && product) return "product";
+    if (pass == 0 && conv_is_product(batch, OC, IC, S, KH, KW, SH, SW, PH, PW, false)) return "product";
     if (pass == 0 && !forward_takes_implicit(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)) return "im2col";
     if (implicit_is_direct(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)) return "direct";
     return cdx::conv_rowwin_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW) ? "rowwin" : "gather";
