@@ -251,7 +251,10 @@ size_t forward_workspace(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int6
 // for up to 16 rows needs scratch that a convolution's caller does not bring:
 // those stay with the implicit kernels, whose waves split k (1 x 2048 -> 64, 28^2
 // 20 us against 24 with the scratch allocated; 2048 -> 512, 7^2 17 against 25;
-// 4096 -> 64, 28^2 38 against 24).
+// 4096 -> 64, 28^2 38 against 24).  So does backward data of one image, up to 16
+// channels to many: the product's kernel for up to 16 k is slow on many short
+// rows (8 -> 2048 channels, 13^2 12.0 us against 7.8, 16 -> 2048, 40^2 14.0
+// against 11.9; 16 -> 32, 224^2 7.4 against 10.9).
 cdx::GemmArgs product_args(const float* w, int64_t rows, int64_t depth, const float* in,
                            const float* bias, float* out, int64_t batch, int64_t S, bool two_level) {
     cdx::GemmArgs g{CDX_OP_N, CDX_OP_N, rows, S, depth, w, depth, in, S, out, S, 0, 0, bias,
@@ -266,7 +269,7 @@ cdx::GemmArgs product_args(const float* w, int64_t rows, int64_t depth, const fl
 bool conv_is_product(int64_t batch, int64_t rows, int64_t depth, int64_t S, int64_t KH, int64_t KW,
                      int64_t SH, int64_t SW, int64_t PH, int64_t PW, bool two_level) {
     return KH == 1 && KW == 1 && SH == 1 && SW == 1 && PH == 0 && PW == 0 && rows > 0 && depth > 0 &&
-           batch <= 65535 && S > 0 &&
+           batch <= 65535 && S > 0 && !(two_level && batch == 1 && depth <= 16 && rows >= 1024) &&
            (batch != 1 || cdx::gemm_f32_workspace(product_args(nullptr, rows, depth, nullptr, nullptr,
                                                                nullptr, 1, S, two_level)) == 0);
 }

@@ -101,6 +101,10 @@ def test_conv_implicit(g, want):
     ((2, 256, 8, 28, 28, 3, 3, (1, 1), (1, 1)), "rowwin"),       # k = 72
     ((2, 256, 15, 28, 28, 3, 3, (1, 1), (1, 1)), "direct"),      # k = 135
     ((98, 12, 64, 16, 16, 3, 3, (1, 1), (1, 1)), "direct"),      # 12 channels
+    ((1, 2048, 8, 13, 13, 1, 1), "direct"),                      # 1x1: few to many channels
+    ((2, 2048, 8, 13, 13, 1, 1), "product"),
+    ((1, 32, 16, 224, 224, 1, 1), "product"),
+    ((1, 64, 2048, 20, 20, 1, 1), "direct"),                     # k-slices
 ])
 def test_conv_backward_data(g, want):
     assert conv_kernel("data", *g) == want
