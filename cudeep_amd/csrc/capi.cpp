@@ -1376,11 +1376,16 @@ extern "C" const char* cdxi_gemm_kernel(int in, int opA, int opB, int64_t M, int
 }
 
 // Internal: the kernel of a convolution.  `pass`: 0 cdx_conv2d_forward_f32, 1
-// cdx_conv2d_forward_implicit_f32, 2 cdx_conv2d_backward_data_f32.
+// cdx_conv2d_forward_implicit_f32, 2 cdx_conv2d_backward_data_f32, 3
+// cdx_conv2d_backward_weight_f32.
 extern "C" const char* cdxi_conv_kernel(int pass, int64_t batch, int64_t IC, int64_t OC, int64_t IH,
                                         int64_t IW, int64_t KH, int64_t KW, int64_t SH, int64_t SW,
                                         int64_t PH, int64_t PW) {
     const int64_t S = conv_out(IH, KH, SH, PH) * conv_out(IW, KW, SW, PW);
+    if (pass == 3)
+        return cdx::conv_wgrad_implicit_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)
+                   ? cdx::conv_wgrad_kernel_name(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)
+                   : "columns";
     if (pass == 2) {
         if (!bwd_data_rowwin(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)) return "columns";
         if (conv_is_product(batch, IC, OC, S, KH, KW, SH, SW, PH, PW, true)) return "product";

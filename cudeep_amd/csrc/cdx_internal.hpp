@@ -251,10 +251,16 @@ int launch_conv_wgrad_f32(const float* dy, const float* x, float* dw, float* ws,
                           int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH, int64_t KW,
                           int64_t SH, int64_t SW, int64_t PH, int64_t PW, hipStream_t stream);
 
+// The kernel that launch_conv_wgrad_f32 runs (for tests that aim at one).
+const char* conv_wgrad_kernel_name(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
+                                   int64_t KH, int64_t KW, int64_t SH, int64_t SW, int64_t PH,
+                                   int64_t PW);
+
 // The same without LDS staging (conv_wgrad_direct.hip): out is
 // [slices][OC][IC*KH*KW] partials, or dw itself for one slice.
 bool conv_wgrad_direct_ok(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH,
                           int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW);
+int conv_wgrad_direct_fm(int64_t OC);   // channels per wave, in sixteens
 int launch_conv_wgrad_direct_f32(const float* dy, const float* x, float* out, int slices,
                                  int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
                                  int64_t KH, int64_t KW, int64_t SH, int64_t SW, int64_t PH,

@@ -798,22 +798,53 @@ void launch_rows(const RwPlan& r, dim3 grid, dim3 b16, dim3 b64, const RwArgs& p
 }  // namespace
 
 // Where the kernel without LDS staging (conv_wgrad_direct.hip) is the faster
-// one, on the same slices: small layers, whose staged tiles are too few to
-// cover their own latencies; output rows that fill less than half of a row
-// segment; channel counts that pad a 64-channel tile; 1x1 layers, whose filter
-// elements it reads 16 bytes at a time.  Staged / direct, us:
-//   rows kernel   1 x 16 -> 128, 7^2      21 / 8     4 x 64 -> 64, 28^2 (0.23 GFLOP)   19 / 15
-//                 16 x 128 -> 128, 14^2   42 / 33    32 x 256 -> 256, 14^2            207 / 148
-//                 8 x 24 -> 50, 60^2 (0.62 GFLOP) 30 / 34     32 x 64 -> 64, 56^2      86 / 130
-//   gather kernel 6 x 56 -> 46, 31^2, 3x3 s2      29 / 13     8 x 64 -> 128, 56^2, s2  33 / 29
-//                 20 x 128 -> 168, 28^2, 7x7 s2  200 / 161    16 x 16 -> 32, 112^2, 5x5 199 / 129
-//                 1 x 76 -> 128, 60^2, 7x7        63 / 67     16 x 3 -> 64, 224^2, 7x7 s2 84 / 88
-//   1x1           16 x 256 -> 64, 56^2            49 / 43     8 x 128 -> 64, 31^2       31 / 14
+// one, on the same slices.  Staged / direct, us:
+//   1x1 layers, whose filter elements it reads 16 bytes at a time: all
+//     8 x 128 -> 64, 31^2 29 / 13       16 x 256 -> 64, 56^2 48 / 41
+//     32 x 1024 -> 1024, 14^2 338 / 172  64 x 512 -> 512, 28^2 (26 GFLOP) 480 / 273
+//   rows kernel, output rows of up to 16 pixels, half a row segment: all
+//     16 x 128 -> 128, 14^2 41 / 32      32 x 512 -> 512, 14^2 (30 GFLOP) 750 / 450
+//     64 x 512 -> 512, 7^2 723 / 293     32 x 1024 -> 1024, 14^2 2916 / 1617
+//   rows kernel, wider rows, up to 0.5 GFLOP, whose staged tiles are too few to
+//   cover their own latencies: while this kernel's workgroups come in two per
+//   CU, or most of a staged tile is padding
+//     1 x 64 -> 64, 56^2 (252) 19 / 13         4 x 64 -> 64, 28^2 (504) 17 / 14
+//     16 x 16 -> 128, 28^2 (1120) 24 / 28      4 x 128 -> 32, 32^2 (1152) 18 / 25
+//     8 x 128 -> 16, 40^2 (1152, pad 1.4 x 4) 41 / 31   16 x 8 -> 16, 112^2 60 / 42
+//     8 x 24 -> 50, 60^2 (0.62 GFLOP) 30 / 34  32 x 64 -> 64, 56^2 86 / 130
+//   gather kernel, up to 1 GFLOP or with output channels that pad its 64 by an
+//   eighth: where its tiles' padding is a third more than this kernel's, or its
+//   workgroups leave CUs idle, or (64-channel waves) this kernel's waves are long
+//     4 x 128 -> 128, 28^2 s2 (36 of 256) 33 / 14   20 x 128 -> 168, 28^2, 7x7 s2 (198) 197 / 163
+//     16 x 16 -> 32, 112^2, 5x5 (pad 2.8) 196 / 129  32 x 32 -> 192, 31^2 s2 (192) 31 / 36
+//     16 x 200 -> 144, 31^2 s2 (240) 53 / 87        32 x 128 -> 160, 56^2, 5x5 (255) 1562 / 1768
+//     16 x 24 -> 56, 224^2, 5x5 (256, 196 steps) 969 / 866
+//     1 x 512 -> 512, 14^2 s2 (one step per wave) 9 / 19
 static bool direct_pays(const WgGeom& g) {
-    const long double flops = 2.0L * g.B * g.S() * g.OC * g.Kc();
     if (g.KH == 1 && g.KW == 1 && g.SH == 1 && g.SW == 1 && g.PH == 0 && g.PW == 0) return true;
-    if (rows_applies(g)) return flops <= 0.5e9L || g.OW <= 16;
-    return flops <= 1e9L || ceil_div(g.OC, WG_BM) * WG_BM * 100 >= g.OC * 112;
+    const double flops = 2.0 * (double)g.B * (double)g.S() * (double)g.OC * (double)g.Kc();
+    const double pad_oc = (double)(ceil_div(g.OC, WG_BM) * WG_BM) / (double)g.OC;
+    const int64_t wave_oc = 16 * conv_wgrad_direct_fm(g.OC);
+    const int64_t tiles = ceil_div(g.Kc(), 32) * ceil_div(g.OC, wave_oc);
+    if (rows_applies(g)) {
+        if (g.OW <= 16) return true;
+        if (flops > 0.5e9) return false;
+        const RwPlan r = rw_plan(g);
+        const double pad_row = (double)(r.nseg * r.bkp) / (double)g.OW;
+        const double pad_ic = (double)(ceil_div(g.IC, r.ict) * r.ict) / (double)g.IC;
+        return tiles * r.splits <= 550 || pad_row >= 1.3 || pad_row * pad_oc * pad_ic >= 5.0;
+    }
+    if (flops > 1e9 && pad_oc < 1.12) return false;
+    const int slices = splits_for(g);
+    const int64_t steps = ceil_div(ceil_div(g.B * ceil_div(g.S(), 16), slices), 4);   // per wave
+    const double pad = pad_oc * (double)(ceil_div(g.Kc(), WG_BN) * WG_BN);
+    const double pad_direct = (double)(ceil_div(g.OC, wave_oc) * wave_oc) / (double)g.OC *
+                              (double)(ceil_div(g.Kc(), 32) * 32);
+    if (pad >= 1.36 * pad_direct) return true;
+    if (steps <= 2 && tiles * slices >= 700) return false;
+    const int64_t wgs = g.tiles() * slices;
+    const double fill = (double)wgs / (double)(ceil_div(wgs, 256) * 256);
+    return flops <= 1e9 ? fill < 0.72 : fill <= 0.85 || (wave_oc == 64 && steps >= 20);
 }
 
 bool conv_wgrad_implicit_ok(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
@@ -834,6 +865,15 @@ size_t conv_wgrad_implicit_floats(int64_t batch, int64_t IC, int64_t OC, int64_t
     const WgGeom g = make_geom(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW);
     const int s = rows_applies(g) ? rw_plan(g).splits : splits_for(g);
     return s > 1 ? (size_t)s * (size_t)OC * (size_t)g.Kc() : 0;
+}
+
+const char* conv_wgrad_kernel_name(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
+                                   int64_t KH, int64_t KW, int64_t SH, int64_t SW, int64_t PH,
+                                   int64_t PW) {
+    const WgGeom g = make_geom(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW);
+    if (direct_pays(g) && conv_wgrad_direct_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW))
+        return "direct";
+    return rows_applies(g) ? "rows" : "gather";
 }
 
 int launch_conv_wgrad_f32(const float* dy, const float* x, float* dw, float* ws, int64_t batch,

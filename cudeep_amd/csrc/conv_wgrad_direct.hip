@@ -210,6 +210,12 @@ void launch_fm(int fm, dim3 grid, hipStream_t stream, const WdArgs& p) {
 
 }  // namespace
 
+// Channels per wave, in sixteens: the most, unless that pads more.
+int conv_wgrad_direct_fm(int64_t OC) {
+    auto padded = [&](int fm) { return ceil_div(OC, 16 * fm) * 16 * fm; };
+    return OC <= 16 ? 1 : padded(2) * 115 < padded(4) * 100 ? 2 : 4;
+}
+
 // 32-bit byte offsets within an image of either tensor, 32-bit steps.
 bool conv_wgrad_direct_ok(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH,
                           int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
@@ -237,9 +243,7 @@ int launch_conv_wgrad_direct_f32(const float* dy, const float* x, float* out, in
     p.steps = (int)(batch * p.spi);
     p.chunk = (int)ceil_div(p.steps, slices);
     p.div_ow = div_magic(OW); p.div_khw = div_magic(KH * KW); p.div_kw = div_magic(KW);
-    auto padded = [&](int fm) { return ceil_div(OC, 16 * fm) * 16 * fm; };
-    int fm = OC <= 16 ? 1 : 4;
-    if (fm == 4 && padded(2) * 115 < padded(4) * 100) fm = 2;
+    const int fm = conv_wgrad_direct_fm(OC);
     const dim3 grid((unsigned)ceil_div(p.Kc, 32), (unsigned)ceil_div(OC, 16 * fm), (unsigned)slices);
     const bool one = KH == 1 && KW == 1 && SH == 1 && SW == 1 && PH == 0 && PW == 0;
     if (one) launch_fm<true>(fm, grid, stream, p);

@@ -15,8 +15,9 @@ def gemm_kernel(kind, M, N, K, tA=False, tB=False, lda=None, ldb=None):
 
 
 def conv_kernel(what, B, IC, OC, H, W, KH, KW, stride=(1, 1), pad=(0, 0)):
-    """`what`: "forward", "implicit" (the implicit forward entry point) or "data" (backward)."""
+    """`what`: "forward", "implicit" (the implicit forward entry point) "data" or "weight"
+    (backward)."""
     f = L.lib().cdxi_conv_kernel
     f.restype, f.argtypes = ctypes.c_char_p, [ctypes.c_int] + [ctypes.c_int64] * 11
-    return f(("forward", "implicit", "data").index(what), B, IC, OC, H, W, KH, KW, *stride,
+    return f(("forward", "implicit", "data", "weight").index(what), B, IC, OC, H, W, KH, KW, *stride,
              *pad).decode()

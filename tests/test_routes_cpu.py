@@ -108,3 +108,25 @@ def test_conv_implicit(g, want):
 ])
 def test_conv_backward_data(g, want):
     assert conv_kernel("data", *g) == want
+
+
+@pytest.mark.parametrize("g,want", [
+    ((64, 512, 512, 28, 28, 1, 1), "direct"),                        # 1x1
+    ((32, 1024, 1024, 14, 14, 3, 3, (1, 1), (1, 1)), "direct"),      # rows of up to 16
+    ((4, 64, 64, 28, 28, 3, 3, (1, 1), (1, 1)), "direct"),           # 504 workgroups
+    ((16, 16, 128, 28, 28, 3, 3, (1, 1), (1, 1)), "rows"),           # 1120
+    ((8, 128, 16, 40, 40, 3, 3, (1, 1), (1, 1)), "direct"),          # rows of 40 in 56
+    ((16, 8, 16, 112, 112, 3, 3, (1, 1), (1, 1)), "direct"),         # mostly padding
+    ((32, 64, 64, 56, 56, 3, 3, (1, 1), (1, 1)), "rows"),            # 7 GFLOP
+    ((4, 128, 128, 28, 28, 3, 3, (2, 2), (1, 1)), "direct"),         # 36 workgroups
+    ((32, 32, 192, 31, 31, 3, 3, (2, 2), (1, 1)), "gather"),         # 192
+    ((16, 16, 32, 112, 112, 5, 5, (1, 1), (2, 2)), "direct"),        # padding
+    ((16, 200, 72, 7, 7, 5, 5, (2, 2), (2, 2)), "direct"),
+    ((16, 200, 144, 31, 31, 3, 3, (2, 2), (1, 1)), "gather"),
+    ((20, 128, 168, 28, 28, 7, 7, (2, 2), (3, 3)), "direct"),        # 198
+    ((16, 24, 56, 224, 224, 5, 5, (1, 1), (2, 2)), "direct"),        # 196 steps per wave
+    ((1, 512, 512, 14, 14, 3, 3, (2, 2), (1, 1)), "gather"),         # one
+    ((16, 3, 64, 224, 224, 7, 7, (2, 2), (3, 3)), "gather"),         # whole channels, 4 GFLOP
+])
+def test_conv_backward_weight(g, want):
+    assert conv_kernel("weight", *g) == want
