@@ -597,14 +597,19 @@ int cdx_conv2d_forward_f32(const float* input, const float* weight, const float*
 
 // A 3x3 stride-1 layer that Winograd's three launches (transforms and 36
 // products, each a pass over memory) do not pay for: up to 1 GFLOP of direct
-// products, with k long enough to split (forward, Winograd against direct, us:
+// products, with k long enough to split and, as every wave walks a quarter of
+// it, no longer than 256 channels (forward, Winograd against direct, us:
 // 1 x 16 -> 128, 7^2 15 / 8; 2 x 62 -> 23, 31^2 18 / 10; 8 x 24 -> 50, 60^2 28
-// / 22; 4 x 128 -> 128, 28^2 25 / 23; 1.85 GFLOP, 8 x 64 -> 64, 56^2 29 / 39).
+// / 22; 4 x 128 -> 128, 28^2 25 / 23; 16 x 32 -> 512, 14^2 31 / 20; 16 x 200 -> 64,
+// 13^2 27 / 22; 2 x 200 -> 96, 20^2 17 / 21; 8 x 256 -> 64, 6^2 20 / 21; 1 x 256
+// -> 16, 28^2 14 / 20; 3 x 512 -> 48, 20^2 24 / 46; 32 x 512 -> 48, 7^2 33 / 47;
+// 1.85 GFLOP, 8 x 64 -> 64, 56^2 29 / 39).  Among 193 to 256 channels either may
+// win; the direct kernel is kept there for its smaller error.
 int cdx_conv2d_3x3_is_small(int64_t batch, int64_t in_channels, int64_t out_channels,
                             int64_t out_h, int64_t out_w) {
     const long double flops = 18.0L * batch * in_channels * out_channels * out_h * out_w;
     return batch > 0 && out_h > 0 && out_w > 0 && out_channels > 0 && in_channels * 9 >= 128 &&
-           flops <= 1e9L;
+           in_channels <= 256 && flops <= 1e9L;
 }
 
 size_t cdx_conv2d_winograd_workspace_size(int64_t batch, int64_t in_channels,

@@ -14,14 +14,15 @@ namespace kernels {
 // launch_conv2d_backward_data_kernel<float>.  Auto follows the reference's
 // forward routing (src/kernels/conv_kernel.cu:242-275) where that pays:
 // Winograd F(4x4, 3x3) for 3x3 stride-1 layers with at least 16 output pixels
-// per image unless they are small (cdx_conv2d_3x3_is_small), the implicit GEMM
-// (or, for 1x1 layers, a product per image) otherwise, im2col + GEMM for the
-// reference's naive shapes; backward data applies the Winograd rule
+// per image unless they are small (cdx_conv2d_3x3_is_small: the implicit GEMM;
+// since that depends on the batch, one image alone and in a larger batch may
+// differ by Winograd's error), cdx_conv2d_forward_f32's choice of implicit GEMM,
+// im2col + GEMM or, for 1x1 layers, a product per image otherwise; backward data applies the Winograd rule
 // to the transposed convolution it runs (3x3, stride 1, padding <= 2, at
 // least 16 input pixels per image) in the TF32 modes, and keeps the GEMM
 // route in FP32 (whose error bound is twice the reference's GEMM + col2im
-// route).  Im2col never takes Winograd (layers other than 3x3 stride 1 still
-// take the implicit GEMM, which needs no column buffer); Implicit forces the
+// route).  Im2col never takes Winograd (layers other than 3x3 stride 1 are still
+// cdx_conv2d_forward_f32's choice); Implicit forces the
 // implicit GEMM forward (backward data as Im2col).  Winograd on another
 // geometry throws.
 enum class ConvAlgorithm { Auto, Im2col, Winograd, Implicit };

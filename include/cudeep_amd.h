@@ -216,8 +216,11 @@ int cdx_im2col_f32(const float* input, float* col,
 
 /* Bytes of workspace cdx_conv2d_forward_f32 needs: the im2col buffer of one
  * round of images (the whole batch while its buffer stays within 128 MiB,
- * else rounds below that sized for whole waves of GEMM tiles), or 0 for
- * layers beyond 4 MiB of columns that form none (see below). */
+ * else rounds below that sized for whole waves of GEMM tiles), or 0 beyond 4 MiB
+ * of columns for layers of K_col >= 9 other than 3x3 stride-1 ones.  Layers
+ * that ask for columns and end on a route without them (below 4 MiB; 1x1 of
+ * fewer than 9 channels) leave the workspace alone: the size depends neither on
+ * the output channels nor on the route. */
 size_t cdx_conv2d_forward_workspace_size(
     int64_t batch, int64_t in_channels, int64_t in_h, int64_t in_w,
     int64_t kernel_h, int64_t kernel_w, int64_t stride_h, int64_t stride_w,
@@ -264,7 +267,10 @@ int cdx_conv2d_forward_implicit_f32(const float* input, const float* weight,
 /* 1 where a 3x3 stride-1 convolution is small enough that the implicit GEMM
  * (forward; for backward data cdx_conv2d_backward_data_f32, asked with the
  * transposed layer's channels and grad_input's size) beats Winograd's three
- * passes, else 0. */
+ * passes, else 0.  It depends on the batch: where the caller leaves the choice
+ * to this (ConvAlgorithm::Auto), one image alone and the same image in a larger
+ * batch can come from different algorithms and differ by Winograd's error (about 4e-5 of
+ * the output's norm in the TF32 modes). */
 int cdx_conv2d_3x3_is_small(int64_t batch, int64_t in_channels, int64_t out_channels,
                             int64_t out_h, int64_t out_w);
 

@@ -130,3 +130,12 @@ def test_conv_backward_data(g, want):
 ])
 def test_conv_backward_weight(g, want):
     assert conv_kernel("weight", *g) == want
+
+
+@pytest.mark.parametrize("g,want", [((1, 16, 128, 7, 7), 1), ((1, 14, 128, 7, 7), 0),
+                                    ((4, 128, 128, 28, 28), 1), ((8, 64, 64, 56, 56), 0),
+                                    ((2, 256, 64, 20, 20), 1), ((2, 257, 64, 20, 20), 0),
+                                    ((3, 512, 48, 20, 20), 0)])
+def test_small_3x3(g, want):
+    from cudeep_amd import _lib as L
+    assert L.lib().cdx_conv2d_3x3_is_small(*g) == want
