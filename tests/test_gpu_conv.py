@@ -181,11 +181,9 @@ IMPLICIT_GEOMS = [  # (B, C, H, W, OC, KH, KW, SH, SW, PH, PW)
     (2, 8, 6, 130, 16, 3, 3, 1, 2, 1, 1),      # pixels not a multiple of the 128 tile
     (1, 37, 12, 12, 65, 2, 2, 2, 2, 0, 0),     # Kc = 148: k-tail, OC = 65
     (2, 16, 14, 14, 64, 3, 3, 1, 1, 1, 1),     # 3x3 stride 1 through the implicit kernel
-    # row-window form: 5 chunks of 8 channels, a 7 x 104 window (3 of 4
-    # positions per thread used), 200 taps per chunk padded to 208
+    # (the layers above and below run on the direct kernel; the row-window form's
+    # windows and 80-, 112- and 128-pixel tiles: test_gpu_conv_tiles.py)
     (2, 40, 12, 100, 24, 5, 5, 1, 1, 2, 2),
-    # enough workgroups that the plan takes 128- and 112-pixel tiles (the
-    # small layers above take 80)
     (48, 8, 20, 32, 16, 3, 3, 1, 1, 1, 1),
     (42, 8, 20, 32, 16, 3, 3, 1, 1, 1, 1),
 ]
@@ -226,10 +224,10 @@ def test_conv_implicit_parity(g):
     (2, 8, 10, 56, 16, 3, 3, 1, 1, 0, 1),     # no vertical padding
 ])
 def test_rowwin_consecutive_pixel_lanes(g):
-    """Stride-1 layers whose output width the row-window kernel's pixel-block
-    count divides: each lane then takes consecutive pixels of one output row
-    and reads them at immediate offsets, with the output tile staged through
-    LDS.  The implicit forward (one-level k sum) and the stride-1 backward
+    """Stride-1 layers at widths that the row-window kernel's pixel-block counts
+    divide.  Layers this small run on the direct kernel; that kernel itself is
+    tested at these widths, and larger, in test_gpu_conv_tiles.py.  The implicit
+    forward (one-level k sum) and the stride-1 backward
     data through the same kernel (two-level sum, the flipped filter) both
     pass the gates of the other geometries: <= 2 x the reference routes'
     errors against fp64."""
@@ -321,7 +319,7 @@ def test_conv_workspace_and_no_bias():
 
 
 @pytest.mark.parametrize("g", [(32, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1),    # C5: rows kernel
-                               (2, 5, 13, 11, 7, 3, 2, 2, 1, 1, 0)])       # gather kernel
+                               (2, 5, 13, 11, 7, 3, 2, 2, 1, 1, 0)])       # direct kernel
 def test_backward_weight_workspace_query_is_what_the_launch_takes(g):
     """cdx_conv2d_backward_weight_workspace_size is the scratch of the route
     the launch takes: a workspace of exactly that size is accepted, one
@@ -395,12 +393,13 @@ BWD_GEOMS = [  # (B, C, H, W, OC, KH, KW, SH, SW, PH, PW)
     (1, 8, 15, 17, 6, 1, 1, 1, 1, 0, 0),
     (2, 3, 6, 7, 4, 3, 3, 1, 1, 3, 0),
     (2, 33, 10, 30, 65, 3, 3, 1, 1, 0, 2),
-    # 3x3 stride 1 row-window weight gradient: rows wider than 64 pixels (two
-    # segments), 61-pixel rows, pad 2 with partial channel tiles
+    # 3x3 stride 1 weight gradients: rows wider than 64 pixels, 61-pixel rows, pad
+    # 2 with partial channel tiles (on the direct kernel, as all of these; the
+    # tiling kernels' own sizes are in test_gpu_conv_tiles.py)
     (1, 4, 5, 70, 8, 3, 3, 1, 1, 1, 1),
     (2, 16, 9, 61, 16, 3, 3, 1, 1, 1, 1),
     (1, 20, 6, 33, 70, 3, 3, 1, 1, 2, 2),
-    # backward data through 128- and 112-pixel row-window tiles
+    # backward data over many pixels, few channels
     (48, 8, 20, 32, 16, 3, 3, 1, 1, 1, 1),
     (42, 8, 20, 32, 16, 3, 3, 1, 1, 1, 1),
 ]

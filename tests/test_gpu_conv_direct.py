@@ -1,6 +1,6 @@
 """Convolutions whose waves gather their own operands (conv_direct.hip) and 1x1 layers as plain
-products: edges of the 32-pixel and 16 / 32 / 64-channel tiles, of the 16-k steps, of the 1024-k
-tables and of the four k runs, padding and strides.  Forward and stride-1 backward data against
+products: edges of the 32-pixel and 16-channel tiles, of the 16-k steps, of the 1024-k tables and of
+the four k runs, padding and strides (32- and 64-channel waves: test_gpu_conv_direct_plans.py).  Forward and stride-1 backward data against
 fp64 within twice the error of the reference's own route (plus one rounding for short sums)."""
 import numpy as np
 import pytest

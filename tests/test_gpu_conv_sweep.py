@@ -1,7 +1,7 @@
 """Seeded random sweep of conv backward weight and data (cdx_conv2d_backward_*
 through cudeep_amd.ops), the im2col forward and the implicit forward: mostly 3x3 stride-1 layers
-with random widths (1 .. 130: one or two row segments of the row-window
-weight-gradient kernel), pads 0 .. 2, channel counts off the 16-channel and
+with random widths (1 .. 130; layers this small run on the direct kernels, the
+tiling ones are swept in test_gpu_conv_tiles.py), pads 0 .. 2, channel counts off the 16-channel and
 64-channel tile sizes, plus other kernel sizes and strides.  FP32 mode gates:
 <= 2 x the error of the reference's routes restated on the CPU (im2col +
 seq-FMA GEMM), against fp64."""
@@ -62,7 +62,7 @@ def test_conv_random_sweep(seed):
         y64 = oracle.conv2d_direct64(x, w, None, st, pd)
         ey_ref = oracle.rel_fro(oracle.conv2d_ref_im2col(x, w, None, st, pd), y64)
         assert oracle.rel_fro(y, y64) <= 2 * ey_ref + 2.0 ** -24, (g, "forward")
-        # implicit forward (the row-window kernel wherever its window fits)
+        # implicit forward
         b = normal(rng, (OC,), 0.1)
         yi = host(o.conv2d_implicit(dev(x), dev(w), dev(b), st, pd))
         yi64 = oracle.conv2d_direct64(x, w, b, st, pd)

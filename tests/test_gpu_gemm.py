@@ -689,7 +689,7 @@ def _classes(C):
 
 @pytest.mark.parametrize("M,N,K,tA,tB", [
     (64, 64, 64, False, False),
-    (300, 200, 784, False, False),       # ragged tiles (bounds-checked kernel)
+    (300, 200, 784, False, False),       # ragged tiles (unstaged kernel)
     (300, 200, 784, True, True),         # both operands transposed
     (128, 128, 4096, False, False),      # split-K slices repair their own k-range
     (4096, 4096, 64, False, False),      # two-group 256 x 256 kernel (four terms: k-alternating)

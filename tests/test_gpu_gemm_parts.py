@@ -1,6 +1,7 @@
-"""The FP32 GEMM on three exact bf16 parts per operand (gemm_parts.hip): the edges of its tiles
-and k-tiles, its k-slices, the ones column, and operands outside the range in which its parts
-are exact (recomputed on the fp32 matrix path).  Bar throughout: relative Frobenius error against
+"""The FP32 GEMM at the sizes of the three-part kernel (gemm_parts.hip): the edges of its tiles and
+k-tiles, its k-slices, the ones column, and operands outside the range in which its parts are
+exact (recomputed on the fp32 matrix path).  Where k is short the product may run on another
+kernel; test_gpu_gemm_parts_edges.py holds sizes that do not.  Bar throughout: relative Frobenius error against
 fp64 within twice that of the reference's sequential fp32 FMA chain on the same operands (plus
 one rounding where K < 64, as for the other FP32 kernels)."""
 import numpy as np

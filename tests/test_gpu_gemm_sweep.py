@@ -1,5 +1,7 @@
 """Seeded random sweep of the GEMM entry point (cdx_gemm_ex_ws through
-cudeep_amd.ops.gemm): shapes 1..300 in each dimension, all four transposes,
+cudeep_amd.ops.gemm): shapes 1..300 in each dimension (the unstaged and narrow
+kernels in every mode; ragged products on the split kernel are in
+test_gpu_gemm_split_ragged.py), all four transposes,
 operands and output as row-strided views of larger buffers (leading dimension
 > row length), every precision mode, bias mode and epilogue.
 

@@ -168,7 +168,7 @@ def test_captured_step_replays_match_eager(prec, forked):
 @pytest.mark.parametrize("prec", [0, 1])
 def test_conv_step_graph_capture_replays(prec):
     """A conv layer's forward (implicit route, no workspace) and backward
-    (data: the flipped-filter row-window kernel, FP32 products in both
+    (data: the flipped filter's implicit convolution, FP32 products in both
     precision modes; weight: implicit kernel with its split partials; bias) on caller
     workspaces, captured once and replayed with new inputs written eagerly
     between replays: every replay equals the eager step bit for bit, and the

@@ -3,8 +3,8 @@
 (cdx_conv2d_backward_weight_f32, workspace NULL): the same kernels on the
 same inputs, so the results must agree bit for bit -- on calls in a row
 whose scratch use shrinks (stale partials of the previous call must not
-leak into the next), on both backward-weight kernels, in every precision
-mode.  Layers whose scratch exceeds the fixed per-GPU array are refused
+leak into the next), on the row-staged and the direct backward-weight kernel, in
+every precision mode.  Layers whose scratch exceeds the fixed per-GPU array are refused
 before any launch."""
 
 import numpy as np
@@ -62,8 +62,8 @@ def test_refuses_layers_beyond_the_scratch_before_any_launch():
 CALLS = [  # (B, C, H, W, OC, KH, KW, SH, SW, PH, PW), in this order
     (128, 64, 32, 32, 64, 3, 3, 1, 1, 1, 1),   # 64-channel row-window tile, 256 slices (36 MiB)
     (32, 64, 56, 56, 64, 3, 3, 1, 1, 1, 1),    # C5: row-window kernel, 64 partial slices
-    (4, 32, 28, 28, 16, 3, 3, 1, 1, 1, 1),     # smaller: fewer, smaller slices
-    (2, 5, 13, 11, 7, 3, 2, 2, 1, 1, 0),       # gather kernel, ragged
+    (4, 32, 28, 28, 16, 3, 3, 1, 1, 1, 1),     # smaller: fewer, smaller slices (direct kernel)
+    (2, 5, 13, 11, 7, 3, 2, 2, 1, 1, 0),       # direct kernel, ragged (gather: test_gpu_conv_tiles.py)
 ]
 
 
