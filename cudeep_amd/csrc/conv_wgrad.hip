@@ -819,7 +819,10 @@ void launch_rows(const RwPlan& r, dim3 grid, dim3 b16, dim3 b64, const RwArgs& p
 //     16 x 16 -> 32, 112^2, 5x5 (pad 2.8) 196 / 129  32 x 32 -> 192, 31^2 s2 (192) 31 / 36
 //     16 x 200 -> 144, 31^2 s2 (240) 53 / 87        32 x 128 -> 160, 56^2, 5x5 (255) 1562 / 1768
 //     16 x 24 -> 56, 224^2, 5x5 (256, 196 steps) 969 / 866
-//     1 x 512 -> 512, 14^2 s2 (one step per wave) 9 / 19
+//     1x1 with a stride: idle CUs, or a padding of 1.45 (4.5 in narrower waves)
+//     8 x 98 -> 152, 112^2 s2 41 / 65          64 x 200 -> 168, 56^2 s2 153 / 123
+//     1 x 512 -> 512, 14^2 s2 (one step per wave, 2.4 M elements) 9 / 19
+//     1 x 227 -> 120, 13^2, 7x7 s2 (1.3 M) 9 / 13   1 x 204 -> 136, 7^2, 5x5 s2 (0.7 M) 5.7 / 4.5
 static bool direct_pays(const WgGeom& g) {
     if (g.KH == 1 && g.KW == 1 && g.SH == 1 && g.SW == 1 && g.PH == 0 && g.PW == 0) return true;
     const double flops = 2.0 * (double)g.B * (double)g.S() * (double)g.OC * (double)g.Kc();
@@ -840,10 +843,12 @@ static bool direct_pays(const WgGeom& g) {
     const double pad = pad_oc * (double)(ceil_div(g.Kc(), WG_BN) * WG_BN);
     const double pad_direct = (double)(ceil_div(g.OC, wave_oc) * wave_oc) / (double)g.OC *
                               (double)(ceil_div(g.Kc(), 32) * 32);
-    if (pad >= 1.36 * pad_direct) return true;
-    if (steps <= 2 && tiles * slices >= 700) return false;
     const int64_t wgs = g.tiles() * slices;
     const double fill = (double)wgs / (double)(ceil_div(wgs, 256) * 256);
+    if (g.KH * g.KW == 1)
+        return fill < 0.72 || pad >= (wave_oc == 64 ? 1.45 : 4.5) * pad_direct;
+    if (pad >= 1.36 * pad_direct) return true;
+    if (steps <= 1 && (double)g.OC * (double)g.Kc() * slices >= 1e6) return false;
     return flops <= 1e9 ? fill < 0.72 : fill <= 0.85 || (wave_oc == 64 && steps >= 20);
 }
 

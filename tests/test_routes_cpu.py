@@ -122,7 +122,13 @@ def test_conv_backward_data(g, want):
     ((32, 32, 192, 31, 31, 3, 3, (2, 2), (1, 1)), "gather"),         # 192
     ((16, 16, 32, 112, 112, 5, 5, (1, 1), (2, 2)), "direct"),        # padding
     ((16, 200, 72, 7, 7, 5, 5, (2, 2), (2, 2)), "direct"),
+    ((1, 227, 120, 13, 13, 7, 7, (2, 2), (3, 3)), "gather"),         # one step per wave
+    ((1, 204, 136, 7, 7, 5, 5, (2, 2), (2, 2)), "direct"),
     ((16, 200, 144, 31, 31, 3, 3, (2, 2), (1, 1)), "gather"),
+    ((8, 158, 138, 112, 112, 1, 1, (2, 2), (0, 0)), "gather"),       # 1x1 with a stride
+    ((64, 200, 168, 56, 56, 1, 1, (2, 2), (0, 0)), "direct"),
+    ((16, 48, 48, 28, 28, 1, 1, (2, 2), (0, 0)), "direct"),
+    ((8, 177, 256, 7, 7, 5, 5, (2, 2), (2, 2)), "direct"),           # two steps per wave
     ((20, 128, 168, 28, 28, 7, 7, (2, 2), (3, 3)), "direct"),        # 198
     ((16, 24, 56, 224, 224, 5, 5, (1, 1), (2, 2)), "direct"),        # 196 steps per wave
     ((1, 512, 512, 14, 14, 3, 3, (2, 2), (1, 1)), "gather"),         # one
