@@ -215,17 +215,24 @@ bool forward_is_fp32(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int64_t 
 // Of those, the ones on the implicit GEMM.  Below 4 MiB of columns one launch of
 // the direct kernel beats im2col + GEMM as well (6 x 56 -> 46, 31^2, 3x3 stride
 // 2: 16 -> 11 us; 3 x 168 -> 99, 56^2, 1x1 stride 2: 13 -> 9), but not beyond
-// 3200 k, where the column route's product runs in slices (im2col + GEMM /
-// direct: 1 x 128 -> 64, 28^2, 5x5 stride 2, 3200 k 29 / 29; 1 x 200 -> 64, 13^2,
-// 5x5, 5000 k 31 / 44; 2 x 200 -> 48, 14^2, 7x7 stride 2, 9800 k 36 / 84), and
-// not on the kernels that tile larger layers (4 x 256 -> 512, 56^2, 1x1 stride 2
-// 23 / 71; 1 x 128 -> 168, 13^2, 11x11 stride 4 48 / 787).
+// 4000 k, where the column route's product runs in slices (im2col + GEMM /
+// direct: 1 x 128 -> 64, 28^2, 5x5 stride 2, 3200 k 29 / 29; 1 x 75 -> 142, 28^2,
+// 7x7 stride 2, 3675 k 44 / 38; 1 x 200 -> 64, 13^2, 5x5, 5000 k 31 / 44; 2 x 200 ->
+// 48, 14^2, 7x7 stride 2, 9800 k 36 / 84).  The
+// row-window kernel does too where it is preferred to the direct one (7 x 4 ->
+// 200, 60^2, 3x3 stride 2 16 / 8), but for 1x1 layers of 16 channels and more, of
+// whose window it reads all and uses a part (4 x 256 -> 512, 56^2, stride 2 23 / 71, 6
+// x 14 -> 128, 112^2 15 / 12); with more taps than the
+// direct kernel takes columns are faster (1 x 128 -> 168, 13^2, 11x11 stride 4 48 /
+// 787).
 bool forward_takes_implicit(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW,
                             int64_t KH, int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
     return forward_is_fp32(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW) &&
            (!forward_few_columns(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW) ||
-            (IC * KH * KW <= 3200 &&
-             implicit_is_direct(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)));
+            (IC * KH * KW <= 4000 &&
+             cdx::conv_direct_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW) &&
+             (implicit_is_direct(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW) ||
+              ((KH * KW > 1 || IC < 16) && cdx::conv_rowwin_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)))));
 }
 
 // The workspace a forward call asks for: one round of columns, except that of
@@ -251,10 +258,12 @@ size_t forward_workspace(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int6
 // for up to 16 rows needs scratch that a convolution's caller does not bring:
 // those stay with the implicit kernels, whose waves split k (1 x 2048 -> 64, 28^2
 // 20 us against 24 with the scratch allocated; 2048 -> 512, 7^2 17 against 25;
-// 4096 -> 64, 28^2 38 against 24).  So does backward data of one image, up to 16
-// channels to many: the product's kernel for up to 16 k is slow on many short
-// rows (8 -> 2048 channels, 13^2 12.0 us against 7.8, 16 -> 2048, 40^2 14.0
-// against 11.9; 16 -> 32, 224^2 7.4 against 10.9).
+// 4096 -> 64, 28^2 38 against 24).  So do layers of one image, up to 16 channels in
+// the sum and fewer than 56^2 pixels, unless they are fewer than 9 on whole
+// groups of four pixels: the product's kernel for up to 16 k is slow on short
+// rows (forward 16 -> 176, 7^2 11.5 us against 8.0, 16 -> 256, 28^2 7.0 against
+// 3.7; backward data 8 -> 2048, 13^2 12.0 against 7.8; forward 9 -> 512, 56^2 6.9
+// against 8.9, 6 -> 42, 28^2 4.4 against 6.7).
 cdx::GemmArgs product_args(const float* w, int64_t rows, int64_t depth, const float* in,
                            const float* bias, float* out, int64_t batch, int64_t S, bool two_level) {
     cdx::GemmArgs g{CDX_OP_N, CDX_OP_N, rows, S, depth, w, depth, in, S, out, S, 0, 0, bias,
@@ -269,7 +278,7 @@ cdx::GemmArgs product_args(const float* w, int64_t rows, int64_t depth, const fl
 bool conv_is_product(int64_t batch, int64_t rows, int64_t depth, int64_t S, int64_t KH, int64_t KW,
                      int64_t SH, int64_t SW, int64_t PH, int64_t PW, bool two_level) {
     return KH == 1 && KW == 1 && SH == 1 && SW == 1 && PH == 0 && PW == 0 && rows > 0 && depth > 0 &&
-           batch <= 65535 && S > 0 && !(two_level && batch == 1 && depth <= 16 && rows >= 1024) &&
+           batch <= 65535 && S > 0 && !(batch == 1 && depth <= 16 && S < 3136 && (depth >= 9 || S % 4 != 0)) &&
            (batch != 1 || cdx::gemm_f32_workspace(product_args(nullptr, rows, depth, nullptr, nullptr,
                                                                nullptr, 1, S, two_level)) == 0);
 }

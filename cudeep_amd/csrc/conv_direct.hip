@@ -252,18 +252,32 @@ DirectPlan plan_of(int64_t N, int64_t OC, int64_t Kc) {
 // behind: 2 x 12 -> 512, 28^2 10.6 / 12.4, backward data 256 -> 8, 28^2 10.4 /
 // 13.1, 16 x 3 -> 64, 56^2, 5x5 s2 10.2 / 12.8 (with 32 channels 4 x 12 -> 96, 31^2
 // s2 10.9 / 8.7); except for 1x1 layers with a stride, of whose window the
-// row-window kernel uses one pixel in SH SW (4 x 96 -> 100, 56^2 s2 19 / 10).
+// row-window kernel uses one pixel in SH SW (4 x 96 -> 100, 56^2 s2 19 / 10).  Nor
+// do up to eight channels of large filters give that kernel's loop over channel
+// chunks anything to wait for (16 x 8 -> 51, 28^2, 7x7, 112 tiles 18.6 / 23.1; 14 x
+// 8 -> 64, 31^2, 5x5, 121 tiles 12.7 / 14.2), nor up to four at any size (9 x 4 ->
+// 64, 14^2, 5x5 8.7 / 10.8; 1 x 4 -> 81, 56^2, 7x7 12.3 / 14.9).
 // Where that one's window does not fit LDS, its gathering form (64 channels x
 // 128 pixels per workgroup) keeps the layers whose k is not split here (16 x 3
 // -> 64, 224^2, 7x7 stride 2: 73 against 92) and those of 2048 tiles of this
 // kernel and more (2 x 16 -> 168, 224^2, 7x7 s2, 2352 tiles: 132 against 143; 16 x
 // 16 -> 256, 112^2, 7x7 s3, 2888: 144 against 182; 8 x 64 -> 128, 112^2, 7x7 s2,
-// 1568: 370 against 317).
+// 1568: 370 against 317) or eight channels (8 x 8 -> 127, 112^2, 7x7 s2, 1568: 54
+// against 75).  Neither line holds where 64-channel tiles pad a third
+// more than this kernel's waves (9 x 80 -> 81, 112^2, 7x7 s2, 2646: 460 against
+// 329; 16 x 6 -> 24, 31^2, 7x7 21 against 17; a fifth more, 6 x 4 -> 129, 56^2, 7x7 s2
+// 12.5 against 18.4).
 bool conv_direct_pays(int64_t N, int64_t OC, int64_t Kc, int64_t taps, bool rowwin) {
     if (OC <= 16) return true;
     const DirectPlan pl = plan_of(N, OC, Kc);
-    if (ceil_div(OC, 64) * ceil_div(N, 112) < 160) return Kc >= 128 || pl.fm < 4 || taps == 1;
-    return !rowwin && pl.split && ceil_div(N, 32) * ceil_div(OC, 16 * pl.fm) < 2048;
+    const int64_t rw_tiles = ceil_div(OC, 64) * ceil_div(N, 112), waves = ceil_div(OC, 16 * pl.fm);
+    const bool pads_less = ceil_div(OC, 64) * 64 * 3 >= waves * 16 * pl.fm * 4;
+    if (rw_tiles < 160) {
+        if (taps >= 25 && Kc <= 4 * taps) return pads_less;
+        return Kc >= 128 ? Kc > 8 * taps || rw_tiles < 100 || pads_less : pl.fm < 4 || taps == 1;
+    }
+    return !rowwin && pl.split &&
+           ((ceil_div(N, 32) * waves < 2048 && Kc > 8 * taps) || pads_less);
 }
 
 // 32-bit byte offsets into the input and the filter, taps within the mask.

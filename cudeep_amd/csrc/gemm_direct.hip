@@ -215,16 +215,22 @@ int64_t tiles_of(const GemmArgs& g, int64_t side) {
 //   8192 x 256 x 784 NT 38.9      60.6       67.2       31.8
 // so: all products of up to 400 32 x 32 tiles, and beyond that those whose
 // rows or k the tiled kernel would have to check element by element, up to
-// where its larger tiles win even so (k past the last 16 alone costs it least;
-// a short k and a transposed A cost this kernel most; M or N up to 64 has its
-// own wide tiles there).  Tiled / this, us:
-//   1600 x 1600 x 300 NT 32.1 / 28.4 (1600 tiles)   1999 x 1501 x 701 NT   89.7 / 56.3 (2961)
-//   1601^2 x 61 NN       15.9 / 13.5 (2601)         1999 x 1501 x 701 TN   66.9 / 66.9
-//   1601^2 x 127 NT      19.6 / 23.2                8192 x 300 x 100 TN    13.2 / 16.4 (2560)
-//   4160 x 384 x 680 TN  33.8 / 37.8 (1560)         61 x 100001 x 300 NN   61.9 / 91.0 (6252)
-//   548 x 4441 x 120 NN  16.7 / 15.5 (2502)         14912 x 196 x 2302 NN  235 / 177 (3262)
+// where its larger tiles win even so (soonest where k past the last 16 is all
+// that it has to check, for a short k, a transposed A, and M or N up to 64,
+// which has its own wide tiles there; NT below 128 k by the parity of its 16-k
+// steps).  Tiled / this, us (tiles):
+//   1200 x 1200 x 300 NT 21.2 / 17.8 (1444)    16896 x 84 x 1564 NT 102 / 68 (1584)
+//   1584 x 1552 x 50 NT  11.8 / 9.0 (2450)     4160 x 384 x 680 TN  33.8 / 37.8 (1560)
+//   1601^2 x 61 NN       15.9 / 13.5 (2601)
+//   1601^2 x 127 NT      19.6 / 23.2           1601^2 x 65 NT       10.5 / 16.0
+//   1368 x 1664 x 153 TT 19.2 / 15.0 (2236)    8192 x 300 x 100 TN  13.2 / 16.4 (2560)
+//   1999 x 1501 x 701 NT 89.7 / 56.3 (2961)    1999 x 1501 x 701 TN 66.9 / 66.9
+//   548 x 4441 x 120 NN  16.7 / 15.5 (2502)    14912 x 196 x 2302 NN 235 / 177 (3262)
+//   61 x 100001 x 300 NN 61.9 / 91.0 (6252)
 //   NCHW map, with the im2col before it: 96 x 13456 x 585 52.8 / 46.6 (1263),
-//   200 x 7688 x 549 49.7 / 52.8 (1687), 256 x 26912 x 459 104.5 / 133.3 (6728)
+//   200 x 7688 x 549 49.7 / 52.8 (1687), 256 x 26912 x 459 104.5 / 133.3 (6728);
+//   only k ragged, 128 x 6272 x 1044 51.5 / 56.5 (784), 96 x 7688 x 1224 64.5 / 56.5
+//   (723: the tiled kernel pads M), 32 x 200704 x 36 40.2 / 34.2 (6272)
 // 64-row NN products and the convolutions' output map keep one k order, that
 // of the tiled kernels, so that the same column of a wider product (another
 // round of images) is the same bits.
@@ -237,15 +243,22 @@ bool gemm_direct_ok(const GemmArgs& g) {
     if (g.batch == 1 && splitk_applies(ceil_div(g.M, 64) * ceil_div(nb, 64), g.K)) return false;
     const int64_t t32 = tiles_of(g, 32);
     if (t32 <= 400) return true;
-    if (t32 > (g.K >= 128 ? 4096 : 3000)) return false;
     const KParams kp = f32::kparams_of(g, g.K);
-    const bool tn = g.opA == CDX_OP_T && g.opB == CDX_OP_N, nt = g.opA == CDX_OP_N && g.opB == CDX_OP_T;
-    if (kp.vec_a && kp.vec_b) return g.K % 16 != 0 && (t32 <= 1024 || (t32 <= 1700 && !tn && g.n_split == 0));
-    if (t32 <= 1700) return true;
-    if (g.n_split > 0 || tn || g.M <= 64 || nb <= 64) return false;
+    if (g.n_split > 0 && g.M <= 32 && t32 <= 8192)   // (64-row tiles at most half used)
+        return g.K % 16 != 0 || !kp.vec_a || !kp.vec_b;
+    if (t32 > (g.K >= 128 ? 4096 : 3000)) return false;
+    const bool nt = g.opA == CDX_OP_N && g.opB == CDX_OP_T;
+    if (kp.vec_a && kp.vec_b) {
+        if (g.n_split > 0) return g.K % 16 != 0 && g.M % 64 != 0 && t32 <= 1200;
+        return g.K % 16 != 0 && t32 <= (nt && g.K >= 384 ? 2200 : 1450);
+    }
+    if (t32 <= (g.n_split > 0 ? 1500 : 1700)) return true;
+    if (g.n_split > 0 || g.M <= 64 || nb <= 64) return false;
     const bool neither = !kp.vec_a && !kp.vec_b;
-    if (g.K < 128) return !nt && (neither || g.K >= 32);
-    return neither || g.opA == CDX_OP_N;
+    if (nt) return g.K >= 128 || (g.K > 48 && ceil_div(g.K, 16) % 2 == 0);
+    if (g.opB == CDX_OP_T) return g.K >= 32 && !kp.vec_b;
+    if (g.opA == CDX_OP_T) return neither && t32 <= 2500;
+    return g.K >= 32 || neither || t32 <= 2500;
 }
 
 // In the TF32 modes (exact fp32 products are inside their error bar): while

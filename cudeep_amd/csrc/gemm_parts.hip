@@ -531,7 +531,7 @@ namespace {
 // the tiled fp32 kernel's rounds of 64 x 64 tiles.  Both costs are in us, from
 // fits to whole tiles with 16-byte rows; A transposed costs this kernel more,
 // ragged sizes and rows cost the tiled one more.  Within an eighth this kernel
-// is taken, for its smaller error.  Tiled / this, us:
+// is taken, for its smaller error (of which 64 k show little).  Tiled / this, us:
 //   4096 x 4096 x 48 NN   37 / 57    2048 x 2304 x 64 NN     11 / 18
 //   2048 x 2048 x 64 NN   10 / 11    2048 x 2304 x 512 NN    46 / 52
 //   2048 x 2048 x 128 NN  14 / 14    2048 x 2304 x 2048 NN  167 / 179
@@ -546,9 +546,10 @@ bool beats_tiled(const GemmArgs& g, int64_t tiles) {
     const double rounds = (double)ceil_div(tiles * g.batch, 256);
     const double rounds64 = (double)ceil_div(ceil_div(g.M, 64) * ceil_div(nb, 64) * g.batch, 256);
     const bool whole = g.M % 64 == 0 && nb % 64 == 0;
-    const double slow = !kp.vec_a && !kp.vec_b ? 1.7 : !kp.vec_a || !kp.vec_b ? 1.35 : g.K % 16 != 0 ? 1.2 : whole ? 1.0 : 1.1;
+    const double slow = !kp.vec_a && !kp.vec_b ? 1.9 : !kp.vec_a || !kp.vec_b ? 1.45
+                        : g.K % 16 != 0 ? 1.25 : whole ? 1.0 : 1.15;
     const double parts = 3.0 + rounds * (5.0 + (g.opA == CDX_OP_T ? 1.5 : 1.25) * (double)ceil_div(g.K, PBK));
-    return parts <= 1.12 * (6.0 + 0.5 * slow * rounds64 * (double)g.K / PBK);
+    return parts <= (g.K > 64 ? 1.12 : 1.0) * (6.0 + 0.5 * slow * rounds64 * (double)g.K / PBK);
 }
 
 }  // namespace

@@ -12,8 +12,8 @@ from tests.routes import conv_kernel
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("g", [(1, 129, 33, 14, 15, 5, 5, (2, 2), (2, 2)),
-                               (2, 70, 48, 9, 9, 7, 7, (2, 2), (3, 3)),
+@pytest.mark.parametrize("g", [(1, 161, 33, 14, 15, 5, 5, (2, 2), (2, 2)),
+                               (2, 82, 48, 9, 9, 7, 7, (2, 2), (3, 3)),
                                (4, 65, 513, 56, 56, 1, 1, (2, 2), (0, 0)),
                                (1, 12, 40, 13, 13, 11, 11, (4, 4), (5, 5))])
 @pytest.mark.parametrize("prec", [0, 1, 2])

@@ -48,7 +48,7 @@ FORWARD = [
     ((48, 8, 24, 20, 32, 3, 3, (1, 1), (1, 1)), "rowwin"),     # 128-pixel tiles
     ((42, 8, 24, 20, 32, 3, 3, (1, 1), (1, 1)), "rowwin"),     # 112
     ((2, 3, 20, 7, 1500, 3, 3, (1, 1), (1, 1)), "gather"),     # rows too wide for a window
-    ((6, 15, 20, 7, 1600, 3, 3, (1, 1), (1, 1)), "gather"),
+    ((6, 15, 60, 7, 1600, 3, 3, (1, 1), (1, 1)), "gather"),
     ((2, 3, 40, 33, 1201, 5, 5, (2, 2), (2, 2)), "gather"),
 ]
 

@@ -28,6 +28,7 @@ def test_gemm16(kind, M, N, K, tA, tB, want):
 @pytest.mark.parametrize("M,N,K,tA,tB,want", [
     (2048, 2048, 48, False, False, "tiled"),      # short k: the pipeline only fills
     (2048, 2048, 128, False, False, "parts"),
+    (5104, 716, 64, True, True, "tiled"),
     (4096, 4096, 48, False, True, "tiled"),
     (4096, 4096, 512, False, True, "parts"),
     (25088, 392, 32, False, False, "tiled"),
@@ -46,15 +47,18 @@ def test_gemm_f32_parts(M, N, K, tA, tB, want):
 @pytest.mark.parametrize("M,N,K,tA,tB,want", [
     (640, 640, 512, False, False, "direct"),      # up to 400 tiles of 32 x 32
     (640, 672, 512, False, False, "tiled"),
-    (1024, 1024, 100, True, False, "direct"),     # only k ragged: 1024 tiles, 1700 unless TN
-    (1280, 1280, 300, False, True, "direct"),
-    (1280, 1280, 300, True, False, "tiled"),
+    (1200, 1200, 100, True, False, "direct"),     # only k ragged: 1450 tiles
     (1600, 1600, 300, False, True, "tiled"),
+    (16896, 84, 1564, False, True, "direct"),     # NT, long k: 2200
     (1301, 1301, 90, True, False, "direct"),      # rows ragged: 1700
     (1601, 1601, 61, False, False, "direct"),     # beyond, by k and orientation
-    (1601, 1601, 127, False, True, "tiled"),
+    (1601, 1601, 61, False, True, "direct"),
+    (1601, 1601, 65, False, True, "tiled"),
     (1601, 1601, 701, False, True, "direct"),
-    (1601, 1601, 701, True, False, "tiled"),
+    (1368, 1664, 153, True, True, "direct"),
+    (1369, 1664, 152, True, True, "tiled"),
+    (1401, 1451, 701, True, False, "direct"),     # 2024 tiles
+    (1601, 1601, 701, True, False, "tiled"),      # 2601
     (61, 100001, 301, False, False, "tiled"),     # one side within 64: wide tiles there
     (100001, 61, 301, False, True, "tiled"),
     (548, 4441, 120, False, False, "direct"),
@@ -71,14 +75,22 @@ def test_gemm_f32_direct(M, N, K, tA, tB, want):
 @pytest.mark.parametrize("g,want", [
     ((6, 56, 46, 31, 31, 3, 3, (2, 2), (1, 1)), "direct"),       # below 4 MiB of columns
     ((3, 168, 99, 56, 56, 1, 1, (2, 2), (0, 0)), "direct"),
-    ((1, 128, 64, 28, 28, 5, 5, (2, 2), (2, 2)), "direct"),      # 3200 k
-    ((1, 129, 64, 28, 28, 5, 5, (2, 2), (2, 2)), "im2col"),
+    ((1, 160, 64, 28, 28, 5, 5, (2, 2), (2, 2)), "direct"),      # 4000 k
+    ((1, 161, 64, 28, 28, 5, 5, (2, 2), (2, 2)), "im2col"),
     ((2, 200, 48, 14, 14, 7, 7, (2, 2), (3, 3)), "im2col"),
-    ((4, 256, 512, 56, 56, 1, 1, (2, 2), (0, 0)), "im2col"),     # row-window tiles enough
+    ((4, 256, 512, 56, 56, 1, 1, (2, 2), (0, 0)), "im2col"),     # row-window tiles enough, but 1x1
+    ((7, 4, 200, 60, 60, 3, 3, (2, 2), (1, 1)), "rowwin"),       # k < 128
+    ((16, 14, 128, 112, 112, 1, 1, (2, 2), (0, 0)), "rowwin"),   # 1x1 of 14 channels
     ((1, 128, 168, 13, 13, 11, 11, (4, 4), (5, 5)), "im2col"),   # more taps than a mask holds
     ((16, 3, 64, 224, 224, 7, 7, (2, 2), (3, 3)), "gather"),     # beyond 4 MiB
     ((2, 16, 16, 12, 12, 3, 3, (1, 1), (1, 1)), "im2col"),       # the Winograd shape
     ((16, 256, 64, 56, 56, 1, 1, (1, 1), (0, 0)), "product"),
+    ((1, 16, 176, 7, 7, 1, 1), "direct"),                        # one image, 16 k, few pixels
+    ((1, 8, 40, 31, 31, 1, 1), "im2col"),
+    ((1, 8, 40, 28, 28, 1, 1), "product"),
+    ((1, 9, 512, 56, 56, 1, 1), "product"),
+    ((1, 17, 176, 7, 7, 1, 1), "product"),
+    ((1, 12, 40, 13, 13, 11, 11, (4, 4), (5, 5)), "im2col"),
 ])
 def test_conv_forward(g, want):
     assert conv_kernel("forward", *g) == want
@@ -90,8 +102,16 @@ def test_conv_forward(g, want):
     ((4, 12, 96, 31, 31, 3, 3, (2, 2), (1, 1)), "direct"),       # 32-channel waves
     ((4, 96, 100, 56, 56, 1, 1, (2, 2), (0, 0)), "direct"),      # 1x1 with a stride
     ((2, 15, 512, 28, 28, 3, 3, (1, 1), (1, 1)), "direct"),      # k = 135
+    ((16, 8, 51, 28, 28, 7, 7, (1, 1), (3, 3)), "rowwin"),       # eight channels, 112 tiles
+    ((16, 9, 51, 28, 28, 7, 7, (1, 1), (3, 3)), "direct"),
+    ((16, 6, 24, 31, 31, 7, 7, (1, 1), (3, 3)), "direct"),       # (pads less)
+    ((6, 4, 129, 56, 56, 7, 7, (2, 2), (3, 3)), "rowwin"),
+    ((9, 4, 64, 14, 14, 5, 5, (1, 1), (2, 2)), "rowwin"),        # four channels
+    ((9, 5, 64, 14, 14, 5, 5, (1, 1), (2, 2)), "direct"),
     ((2, 16, 168, 224, 224, 7, 7, (2, 2), (3, 3)), "gather"),    # 2352 tiles
+    ((9, 80, 81, 112, 112, 7, 7, (2, 2), (3, 3)), "direct"),     # (pads less)
     ((8, 64, 128, 112, 112, 7, 7, (2, 2), (3, 3)), "direct"),    # 1568
+    ((8, 8, 127, 112, 112, 7, 7, (2, 2), (3, 3)), "gather"),     # eight channels
 ])
 def test_conv_implicit(g, want):
     assert conv_kernel("implicit", *g) == want
@@ -104,6 +124,7 @@ def test_conv_implicit(g, want):
     ((1, 2048, 8, 13, 13, 1, 1), "direct"),                      # 1x1: few to many channels
     ((2, 2048, 8, 13, 13, 1, 1), "product"),
     ((1, 32, 16, 224, 224, 1, 1), "product"),
+    ((1, 3, 16, 31, 31, 1, 1), "direct"),
     ((1, 64, 2048, 20, 20, 1, 1), "direct"),                     # k-slices
 ])
 def test_conv_backward_data(g, want):
