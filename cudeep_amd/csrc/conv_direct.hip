@@ -255,8 +255,9 @@ DirectPlan plan_of(int64_t N, int64_t OC, int64_t Kc) {
 // row-window kernel uses one pixel in SH SW (4 x 96 -> 100, 56^2 s2 19 / 10).  Nor
 // do up to eight channels of large filters give that kernel's loop over channel
 // chunks anything to wait for (16 x 8 -> 51, 28^2, 7x7, 112 tiles 18.6 / 23.1; 14 x
-// 8 -> 64, 31^2, 5x5, 121 tiles 12.7 / 14.2), nor up to four at any size (9 x 4 ->
-// 64, 14^2, 5x5 8.7 / 10.8; 1 x 4 -> 81, 56^2, 7x7 12.3 / 14.9).
+// 8 -> 64, 31^2, 5x5, 121 tiles 12.7 / 14.2), nor four, a chunk without
+// padding, at any size (9 x 4 -> 64, 14^2, 5x5 8.7 / 10.8; 1 x 4 -> 81, 56^2, 7x7
+// 12.3 / 14.9; but 8 x 3 -> 64, 31^2, 7x7 s2 13.8 / 12.0).
 // Where that one's window does not fit LDS, its gathering form (64 channels x
 // 128 pixels per workgroup) keeps the layers whose k is not split here (16 x 3
 // -> 64, 224^2, 7x7 stride 2: 73 against 92) and those of 2048 tiles of this
@@ -273,7 +274,7 @@ bool conv_direct_pays(int64_t N, int64_t OC, int64_t Kc, int64_t taps, bool roww
     const int64_t rw_tiles = ceil_div(OC, 64) * ceil_div(N, 112), waves = ceil_div(OC, 16 * pl.fm);
     const bool pads_less = ceil_div(OC, 64) * 64 * 3 >= waves * 16 * pl.fm * 4;
     if (rw_tiles < 160) {
-        if (taps >= 25 && Kc <= 4 * taps) return pads_less;
+        if (taps >= 25 && Kc == 4 * taps) return pads_less;
         return Kc >= 128 ? Kc > 8 * taps || rw_tiles < 100 || pads_less : pl.fm < 4 || taps == 1;
     }
     return !rowwin && pl.split &&

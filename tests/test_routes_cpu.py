@@ -108,6 +108,7 @@ def test_conv_forward(g, want):
     ((6, 4, 129, 56, 56, 7, 7, (2, 2), (3, 3)), "rowwin"),
     ((9, 4, 64, 14, 14, 5, 5, (1, 1), (2, 2)), "rowwin"),        # four channels
     ((9, 5, 64, 14, 14, 5, 5, (1, 1), (2, 2)), "direct"),
+    ((8, 3, 64, 31, 31, 7, 7, (2, 2), (3, 3)), "direct"),
     ((2, 16, 168, 224, 224, 7, 7, (2, 2), (3, 3)), "gather"),    # 2352 tiles
     ((9, 80, 81, 112, 112, 7, 7, (2, 2), (3, 3)), "direct"),     # (pads less)
     ((8, 64, 128, 112, 112, 7, 7, (2, 2), (3, 3)), "direct"),    # 1568
