@@ -188,10 +188,14 @@ bool forward_few_columns(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int6
 // or, where its window does not fit LDS, the gathering one (conv_implicit.hip).
 bool implicit_is_direct(int64_t batch, int64_t IC, int64_t OC, int64_t IH, int64_t IW, int64_t KH,
                         int64_t KW, int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
+    const int64_t N = batch * conv_out(IH, KH, SH, PH) * conv_out(IW, KW, SW, PW);
+    auto pays = [&](bool rowwin) {
+        return cdx::conv_direct_pays(N, OC, IC * KH * KW, KH * KW, rowwin);
+    };
+    // (whether a window fits is a search: asked where it decides)
     return cdx::conv_direct_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW) &&
-           cdx::conv_direct_pays(batch * conv_out(IH, KH, SH, PH) * conv_out(IW, KW, SW, PW), OC,
-                                 IC * KH * KW, KH * KW,
-                                 cdx::conv_rowwin_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW));
+           (pays(true) ||
+            (pays(false) && !cdx::conv_rowwin_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)));
 }
 
 // The forward dispatch below the Winograd route.  The reference sends a layer
@@ -259,11 +263,12 @@ size_t forward_workspace(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int6
 // those stay with the implicit kernels, whose waves split k (1 x 2048 -> 64, 28^2
 // 20 us against 24 with the scratch allocated; 2048 -> 512, 7^2 17 against 25;
 // 4096 -> 64, 28^2 38 against 24).  So do layers of one image, up to 16 channels in
-// the sum and fewer than 56^2 pixels, unless they are fewer than 9 on whole
-// groups of four pixels: the product's kernel for up to 16 k is slow on short
-// rows (forward 16 -> 176, 7^2 11.5 us against 8.0, 16 -> 256, 28^2 7.0 against
-// 3.7; backward data 8 -> 2048, 13^2 12.0 against 7.8; forward 9 -> 512, 56^2 6.9
-// against 8.9, 6 -> 42, 28^2 4.4 against 6.7).
+// the sum and fewer than 56^2 pixels, whose product's kernel is slow on short rows
+// (forward 16 -> 176, 7^2 11.5 us against 8.0, 16 -> 256, 28^2 7.0 against 3.7;
+// backward data 8 -> 2048, 13^2 12.0 against 7.8; but forward 9 -> 512, 56^2 6.9
+// against 8.9), except forward with fewer than 9, where the other route is
+// im2col (8 -> 40, 31^2 9.8 against 8.8 in two launches, and TF32 products in that
+// mode), and backward data with fewer on whole groups of four pixels.
 cdx::GemmArgs product_args(const float* w, int64_t rows, int64_t depth, const float* in,
                            const float* bias, float* out, int64_t batch, int64_t S, bool two_level) {
     cdx::GemmArgs g{CDX_OP_N, CDX_OP_N, rows, S, depth, w, depth, in, S, out, S, 0, 0, bias,
@@ -278,7 +283,7 @@ cdx::GemmArgs product_args(const float* w, int64_t rows, int64_t depth, const fl
 bool conv_is_product(int64_t batch, int64_t rows, int64_t depth, int64_t S, int64_t KH, int64_t KW,
                      int64_t SH, int64_t SW, int64_t PH, int64_t PW, bool two_level) {
     return KH == 1 && KW == 1 && SH == 1 && SW == 1 && PH == 0 && PW == 0 && rows > 0 && depth > 0 &&
-           batch <= 65535 && S > 0 && !(batch == 1 && depth <= 16 && S < 3136 && (depth >= 9 || S % 4 != 0)) &&
+           batch <= 65535 && S > 0 && !(batch == 1 && depth <= 16 && S < 3136 && (depth >= 9 || (two_level && S % 4 != 0))) &&
            (batch != 1 || cdx::gemm_f32_workspace(product_args(nullptr, rows, depth, nullptr, nullptr,
                                                                nullptr, 1, S, two_level)) == 0);
 }
