@@ -61,7 +61,7 @@
 // split and LDS stores.  At the end the groups exchange halves of their sums
 // through LDS and add even + odd k-tiles.
 //
-// Measured: 4096^3 NN 698 us = 197 TFLOP/s against 980 = 140 on the fp32
+// Measured: 4096^3 NN 707-745 us = 185-194 TFLOP/s against 980 = 140 on the fp32
 // matrix path, 3072^3 390 against 454, 2048^3 92 against 131.  Bound by the
 // MFMA slots: without the split and stores 2048^3 takes 85 us, without the
 // global loads 83, without the MFMAs 53 (each measured with the loads issued
