@@ -766,9 +766,10 @@ RwPlan rw_plan_for(const WgGeom& g, int ict) {
 // most 56 pixels) and each slice is at least 16 row segments long: its
 // partials are four times the 16-channel form's (the whole 64 x 9 IC tile
 // per workgroup), which the slice's work has to outweigh.  Measured on
-// MI355X with the reduction: 64 x 128 x 56^2 552 against 626 us, 32 x 512
-// x 14^2 704 against 862, 32 x 256 x 28^2 357 against 445; C5 (7 row
-// segments per slice) 96 against 93, so C5 keeps the 16-channel tile.
+// MI355X with the reduction: 64 x 128 x 56^2 552 against 626 us, 32 x 256
+// x 28^2 357 against 445; C5 (7 row segments per slice) 96 against 93, so
+// C5 keeps the 16-channel tile.  (Rows of up to 16 pixels are planned here
+// too, but only for their slices: direct_pays takes them.)
 RwPlan rw_plan(const WgGeom& g) {
     if (g.IC % 64 == 0 && rw_bkp(g.OW) <= 56) {
         const RwPlan r = rw_plan_for(g, 64);
