@@ -239,8 +239,36 @@ bool forward_takes_implicit(int64_t batch, int64_t IC, int64_t OC, int64_t IH, i
               ((KH * KW > 1 || IC < 16) && cdx::conv_rowwin_ok(batch, IC, OC, IH, IW, KH, KW, SH, SW, PH, PW)))));
 }
 
-// The workspace a forward call asks for: one round of columns, except that of
-// layers whose whole column buffer would exceed 4 MiB and that never form it.
+// weight[OC, Kc] * col[Kc, ns] -> NCHW: addr = oc*S + (n/S)*OC*S + n%S
+cdx::GemmArgs column_product(int64_t OC, int64_t ns, int64_t Kc, int64_t S, const float* weight,
+                             const float* col, const float* bias, float* output) {
+    return {CDX_OP_N, CDX_OP_N, OC, ns, Kc, weight, Kc > 0 ? Kc : 1, col, ns, output, S, S, OC * S,
+            bias, bias ? CDX_BIAS_ROW : CDX_BIAS_NONE, CDX_EPI_NONE};
+}
+
+// Room behind the columns for the slices of their product, where a layer that
+// no implicit kernel's limits kept from it takes the column route for its long
+// k: the most over the output channels, which the size query does not see
+// (whole 64-row tiles need the most of each count; 25 MB at most).
+constexpr size_t kSliceAlign = 256;
+size_t few_columns_slices(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int64_t KH, int64_t KW,
+                          int64_t SH, int64_t SW, int64_t PH, int64_t PW) {
+    const int64_t Kc = IC * KH * KW;
+    if (Kc < 2048 || batch <= 0 || !forward_few_columns(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW) ||
+        !forward_is_fp32(batch, IC, IH, IW, KH, KW, SH, SW, PH, PW) ||
+        (Kc <= 4000 && cdx::conv_direct_ok(batch, IC, 1, IH, IW, KH, KW, SH, SW, PH, PW)) ||
+        (batch > 1 && KH * KW == 1 && SH == 1 && SW == 1 && PH == 0 && PW == 0))   // a product
+        return 0;
+    const int64_t S = conv_out(IH, KH, SH, PH) * conv_out(IW, KW, SW, PW), ns = batch * S;
+    size_t most = 0;
+    for (int64_t M = 64; cdx::splitk_applies(M / 64 * cdx::ceil_div(ns, (int64_t)64), Kc); M += 64)
+        most = std::max(most, cdx::gemm_f32_workspace(column_product(M, ns, Kc, S, nullptr, nullptr,
+                                                                     nullptr, nullptr)));
+    return most > 0 ? most + kSliceAlign : 0;
+}
+
+// The workspace a forward call is held to: one round of columns, except that
+// of layers whose whole column buffer would exceed 4 MiB and that never form it.
 // (Layers of fewer columns that no longer form them keep asking for it, so
 // that a caller's check of the size stays what it was.)
 size_t forward_workspace(int64_t batch, int64_t IC, int64_t IH, int64_t IW, int64_t KH, int64_t KW,
@@ -474,7 +502,9 @@ size_t cdx_conv2d_forward_workspace_size(int64_t batch, int64_t in_channels, int
                    kernel_h, kernel_w, stride_h, stride_w, pad_h, pad_w))
         return 0;
     return forward_workspace(batch, in_channels, in_h, in_w, kernel_h, kernel_w, stride_h, stride_w,
-                             pad_h, pad_w);
+                             pad_h, pad_w) +
+           few_columns_slices(batch, in_channels, in_h, in_w, kernel_h, kernel_w, stride_h,
+                              stride_w, pad_h, pad_w);
 }
 
 int cdx_conv2d_forward_implicit_f32(const float* input, const float* weight, const float* bias,
@@ -550,11 +580,21 @@ int conv_forward_im2col(const float* input, const float* weight, const float* bi
                                         stride_w, pad_h, pad_w, stream);
         }
         if (!st) {
-            // weight[OC, Kc] * col[Kc, nb*S] -> NCHW: addr = oc*S + (n/S)*OC*S + n%S
-            cdx::GemmArgs g{CDX_OP_N, CDX_OP_N, out_channels, ns, Kc, weight, Kc > 0 ? Kc : 1,
-                            col, ns, output + b0 * out_channels * S, S, S, out_channels * S,
-                            bias, bias ? CDX_BIAS_ROW : CDX_BIAS_NONE, CDX_EPI_NONE};
+            cdx::GemmArgs g = column_product(out_channels, ns, Kc, S, weight, col, bias,
+                                             output + b0 * out_channels * S);
             g.blocked_sum = blocked_sum;
+            // slices go behind the columns where the caller's workspace has the room
+            // (else they are allocated stream-ordered)
+            if (workspace && precision == CDX_PREC_FP32) {
+                const uintptr_t w = (uintptr_t)workspace;
+                const uintptr_t rest = (w + need + kSliceAlign - 1) / kSliceAlign * kSliceAlign;
+                const size_t slices = cdx::gemm_f32_workspace(g);
+                if (slices > 0 && rest - w <= workspace_bytes &&
+                    slices <= workspace_bytes - (rest - w)) {
+                    g.ws = reinterpret_cast<void*>(rest);
+                    g.ws_bytes = workspace_bytes - (rest - w);
+                }
+            }
             st = run_gemm(precision, g, stream);
         }
     }

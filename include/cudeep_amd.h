@@ -220,7 +220,10 @@ int cdx_im2col_f32(const float* input, float* col,
  * of columns for layers of K_col >= 9 other than 3x3 stride-1 ones.  Layers
  * that ask for columns and end on a route without them (below 4 MiB; 1x1 of
  * fewer than 9 channels) leave the workspace alone: the size depends neither on
- * the output channels nor on the route. */
+ * the output channels nor on the route.  Layers of up to 4 MiB of columns whose
+ * product runs in k-slices for its long k (beyond 4000, or a filter of more than 63 taps)
+ * ask for the slices' room too (up to 25 MB); the columns alone are accepted,
+ * and the slices then allocated stream-ordered. */
 size_t cdx_conv2d_forward_workspace_size(
     int64_t batch, int64_t in_channels, int64_t in_h, int64_t in_w,
     int64_t kernel_h, int64_t kernel_w, int64_t stride_h, int64_t stride_w,

@@ -1,6 +1,7 @@
 """The kernels that the library chooses (no GPU needed): both sides of each line."""
 import pytest
 
+from cudeep_amd import _lib as L
 from tests.routes import conv_kernel, gemm_kernel
 
 
@@ -167,3 +168,33 @@ def test_conv_backward_weight(g, want):
 def test_small_3x3(g, want):
     from cudeep_amd import _lib as L
     assert L.lib().cdx_conv2d_3x3_is_small(*g) == want
+
+
+@pytest.mark.parametrize("g", [(1, 161, 14, 15, 5, 5, (2, 2), (2, 2)), (2, 82, 9, 9, 7, 7, (2, 2), (3, 3)),
+                               (1, 40, 13, 13, 11, 11, (4, 4), (5, 5)), (1, 4100, 9, 8, 1, 1, (1, 1), (0, 0))])
+def test_columns_of_a_long_k_have_room_for_slices(g):
+    """The forward query covers the column buffer and the slices of the columns' product, for any
+    number of output channels."""
+    lib = L.lib()
+    B, IC, H, W, KH, KW, (sh, sw), (ph, pw) = g
+    K, ns = IC * KH * KW, B * ((H + 2 * ph - KH) // sh + 1) * ((W + 2 * pw - KW) // sw + 1)
+    got = lib.cdx_conv2d_forward_workspace_size(B, IC, H, W, KH, KW, sh, sw, ph, pw)
+    tiles_n, most = -(-ns // 64), 0
+    for OC in range(17, 64 * (127 // tiles_n) + 1):
+        assert conv_kernel("forward", B, IC, OC, H, W, KH, KW, (sh, sw), (ph, pw)) == "im2col"
+        if lib.cdx_gemm_workspace_size(0, 0, 0, OC, ns, K) > 0:
+            # (64-row tiles, 128 x 64 from 128 rows on; about 768 slices of tiles of 256 k or more)
+            tiles = -(-OC // (128 if OC >= 128 else 64)) * tiles_n
+            s = min((768 + tiles // 2) // tiles, K // 256)
+            chunk = -(-(-(-K // s)) // 16) * 16
+            most = max(most, -(-K // chunk) * OC * ns * 4)
+    assert most > 0 and got >= 4 * K * ns + 255 + most
+
+
+@pytest.mark.parametrize("g", [(1, 160, 28, 28, 5, 5, (2, 2), (2, 2)), (2, 3, 9, 9, 3, 3, (1, 1), (1, 1)),
+                               (2, 5000, 5, 5, 1, 1, (1, 1), (0, 0))])
+def test_other_layers_ask_for_columns_only(g):
+    B, IC, H, W, KH, KW, (sh, sw), (ph, pw) = g
+    ns = B * ((H + 2 * ph - KH) // sh + 1) * ((W + 2 * pw - KW) // sw + 1)
+    assert L.lib().cdx_conv2d_forward_workspace_size(B, IC, H, W, KH, KW, sh, sw, ph, pw) \
+        == 4 * IC * KH * KW * ns
